@@ -25,6 +25,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ptf {
 
 template <typename T>
@@ -371,8 +373,10 @@ __device__ __forceinline__ void fft_passes(cpx<T> (&a)[E], cpx<T>* lds, const La
 // must call it.  wave = true (every line of the block within one wavefront, lines never
 // sharing LDS entries) orders the exchanges per wavefront instead (lds_sync); then a
 // twiddle table in LDS must be complete before the call.  TWH: tw holds only the first
-// LT/2 entries, the others follow from tw[k + LT/2] = -tw[k].
-template <typename T, int N, int R, int DIR, class Lay, bool TWH = false>
+// LT/2 entries, the others follow from tw[k + LT/2] = -tw[k].  LEAN: the transform computes its
+// LDS and twiddle addresses anew instead of sharing them with the kernel's other transforms,
+// which would keep all of them in registers (see fft_lean).
+template <typename T, int N, int R, int DIR, class Lay, bool TWH = false, bool LEAN = false>
 __device__ __forceinline__ void line_fft(cpx<T> (&a)[R], cpx<T>* lds, const Lay& lay, int c, int j,
                                          const cpx<T>* __restrict__ tw, int twstride,
                                          bool wave = false) {
@@ -382,9 +386,20 @@ __device__ __forceinline__ void line_fft(cpx<T> (&a)[R], cpx<T>* lds, const Lay&
   if constexpr (pl.n == 1) {
     dft<R, DIR>(a);
   } else {
+    if constexpr (LEAN) __asm__ volatile("" : "+v"(j));   // an opaque copy of the lane's index
     fft_passes<T, N, R, DIR, 0, Lay, TWH>(a, lds, lay, c, j, tw, twstride, wave);
   }
 }
+
+// Whether a kernel is built lean: its transforms compute their addresses anew, and its accesses
+// share one lane offset (lane_at).  With 10 and more elements per lane, and in the builds with a
+// tightened register budget where the addresses would cost occupancy or spills: all FP32 ones and
+// FP64 from 8 elements (256-point fused z kernel: 168 VGPRs and 76 bytes of spills -> 127 and
+// none, isolated stages at 256^3 1.09-1.10 times as fast; FP32 128^3 ETDRK4 stages 22 -> 18 us).
+// Builds that have registers to spare keep the addresses: a small launch is a chain of
+// latencies, to which the recomputation adds 5 %.
+template <typename T, int R, int OCC>
+constexpr bool fft_lean() { return R >= 10 || (OCC > 0 && R * (int)sizeof(cpx<T>) >= (sizeof(T) == 4 ? 32 : 128)); }
 
 // --------------------------------------------------------------------------
 // linear operator and stage updates
@@ -427,6 +442,34 @@ __device__ __forceinline__ double linear_op(const GridInfo& g, const OpParams& p
 }
 
 enum { EPI_STORE = 0, EPI_RK4 = 1, EPI_ETDRK4 = 2 };
+
+// Element `off` of a block-uniform array.  LEAN (see fft_lean): the byte offset stays in 32
+// bits, so the access takes its base from scalar registers and one vector register of offset
+// for all accesses of a lane, not a 64-bit vector address each.  (A lane's offset spans at most
+// its wavefront's part of a line, see col_kernel: below 4 GiB for every field that fits the
+// device.)
+template <bool LEAN = false, typename X>
+__device__ __forceinline__ X* lane_at(X* base, uint32_t off) {
+  if constexpr (LEAN) {
+    using G = __attribute__((address_space(1))) X;
+    using C = __attribute__((address_space(1))) char;
+    uintptr_t b = reinterpret_cast<uintptr_t>(base);
+    // the base as a scalar value of its own: neither folded into the offset nor kept live
+    __asm__ volatile("" : "+s"(b));
+    return (X*)(G*)((C*)b + (uint32_t)(off * (uint32_t)sizeof(X)));
+  } else {
+    return base + off;
+  }
+}
+
+// A block-uniform pointer (one that came out of a select or a loop) as a scalar value.
+template <typename X>
+__device__ __forceinline__ X* uniform_ptr(X* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<X*>((uint64_t)hi << 32 | lo);
+}
 
 // Non-temporal access to fields that are touched once per stage and not again until
 // the next stage, long after the caches have turned over (the stage state, the
@@ -559,31 +602,31 @@ struct Rk4Ops {
 // one straight-line block); ST = -1 reads it from the arguments.  store = false (lanes
 // of a tail column that only computes) suppresses the state stores.  NTS: the state
 // loads are non-temporal (the caller's blocks cover whole 128-byte lines of the state).
-template <typename T, int ST = -1, bool NTS = true>
+template <typename T, int ST = -1, bool NTS = true, bool LEAN = false>
 __device__ __forceinline__ Rk4Ops<T> rk4_load(const StageArgs<T>& a, long long ubase, uint32_t off) {
   const int stage = ST >= 0 ? ST : a.stage;
   // every field is defined on every path so that the value stays in registers
   const cpx<T> z = {(T)0, (T)0};
   Rk4Ops<T> o = {z, z, z, z};
   if (stage == 0) {
-    o.x = ld_pol<NTS>(a.sol + ubase + off);
+    o.x = ld_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off));
   } else if (stage == 1) {
-    o.s = ld_pol<NTS>(a.sol + ubase + off);
-    o.ac = ld_pol<NTS>(a.acc + ubase + off);
+    o.s = ld_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off));
+    o.ac = ld_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off));
   } else {
-    o.x = ld_pol<NTS>(a.stg + ubase + off);
-    o.s = ld_pol<NTS>(a.sol + ubase + off);
+    o.x = ld_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off));
+    o.s = ld_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off));
     // the compensated low part exists only in the mixed (FP32) form
     constexpr bool kMixed = sizeof(T) == 4;
-    if (stage == 2 || (kMixed && a.sol_lo)) o.ac = ld_pol<NTS>(a.acc + ubase + off);
-    if (kMixed && stage == 3 && a.sol_lo) o.lo = ld_pol<NTS>(a.sol_lo + ubase + off);
+    if (stage == 2 || (kMixed && a.sol_lo)) o.ac = ld_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off));
+    if (kMixed && stage == 3 && a.sol_lo) o.lo = ld_pol<NTS>(lane_at<LEAN>(a.sol_lo + ubase, off));
   }
   return o;
 }
 
 // rk4_finish with the element's linear operator L already evaluated (a caller that
 // updates the same elements in every stage computes it once)
-template <typename T, int ST = -1, bool NTS = true>
+template <typename T, int ST = -1, bool NTS = true, bool LEAN = false>
 __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long ubase, uint32_t off,
                                                T L, int ikx, int iky, int ikz, cpx<T> N,
                                                const Rk4Ops<T>& o, bool store = true) {
@@ -596,24 +639,24 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
   if (stage == 0) {
     const cpx<T> nx = {x.re + h2 * rhs.re, x.im + h2 * rhs.im};
     if (store) {
-      if (a.store_x) st_pol<NTS>(a.stg + ubase + off, nx);
-      st_pol<NTS>(a.acc + ubase + off, rhs);
+      if (a.store_x) st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), nx);
+      st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), rhs);
     }
     return nx;
   } else if (stage == 1) {
     const cpx<T> nx = {o.s.re + h2 * rhs.re, o.s.im + h2 * rhs.im};
     if (store) {
-      st_pol<NTS>(a.stg + ubase + off, nx);
-      st_pol<NTS>(a.acc + ubase + off, {o.ac.re / (T)6 + rhs.re / (T)3, o.ac.im / (T)6 + rhs.im / (T)3});
+      st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), nx);
+      st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), {o.ac.re / (T)6 + rhs.re / (T)3, o.ac.im / (T)6 + rhs.im / (T)3});
     }
     return nx;
   } else if (stage == 2) {
     const cpx<T> nx = {o.s.re + dt * rhs.re, o.s.im + dt * rhs.im};
     const cpx<T> tot = {o.ac.re + rhs.re / (T)3, o.ac.im + rhs.im / (T)3};
     if (store) {
-      st_pol<NTS>(a.stg + ubase + off, nx);
-      if (sizeof(T) == 4 && a.sol_lo) st_pol<NTS>(a.acc + ubase + off, tot);
-      else st_pol<NTS>(a.sol + ubase + off, {o.s.re + dt * tot.re, o.s.im + dt * tot.im});
+      st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), nx);
+      if (sizeof(T) == 4 && a.sol_lo) st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), tot);
+      else st_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off), {o.s.re + dt * tot.re, o.s.im + dt * tot.im});
     }
     return nx;
   } else {
@@ -624,7 +667,7 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
         const T f = (T)filter_value(a.g, a.f_order, a.f_innerK, a.f_decay, ikx, iky, ikz);
         ns = {f * ns.re, f * ns.im};
       }
-      if (store) st_pol<NTS>(a.sol + ubase + off, ns);
+      if (store) st_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off), ns);
       return ns;
     }
     // compensated accumulation: (hi, lo) += dt tot with TwoSum + renormalisation
@@ -642,8 +685,8 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
       li_ = (T)(xi - (double)hi_);
     }
     if (store) {
-      st_pol<NTS>(a.sol + ubase + off, {hr, hi_});
-      st_pol<NTS>(a.sol_lo + ubase + off, {lr, li_});
+      st_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off), {hr, hi_});
+      st_pol<NTS>(lane_at<LEAN>(a.sol_lo + ubase, off), {lr, li_});
     }
     return {hr, hi_};
   }
@@ -651,11 +694,11 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
 
 // op = the member's operator coefficients (a.op[member]), read once by the caller: a
 // read through a.op between the state stores would be repeated for every element.
-template <typename T, int ST = -1, bool NTS = true>
+template <typename T, int ST = -1, bool NTS = true, bool LEAN = false>
 __device__ __forceinline__ cpx<T> rk4_finish(const StageArgs<T>& a, long long ubase, uint32_t off,
                                              const OpParams& op, int ikx, int iky, int ikz, cpx<T> N,
                                              const Rk4Ops<T>& o, bool store = true) {
-  return rk4_finish_L<T, ST, NTS>(a, ubase, off, (T)linear_op(a.g, op, a.nkappah, ikx, iky, ikz), ikx,
+  return rk4_finish_L<T, ST, NTS, LEAN>(a, ubase, off, (T)linear_op(a.g, op, a.nkappah, ikx, iky, ikz), ikx,
                              iky, ikz, N, o, store);
 }
 
@@ -670,7 +713,7 @@ struct EtdOps {
 
 // NTS, NTC: the loads of the state and of the (FP64 real) coefficients are non-temporal
 // (as for rk4_load: where the caller's blocks cover whole 128-byte lines of them)
-template <typename T, int ST = -1, bool NTS = true, bool NTC = true>
+template <typename T, int ST = -1, bool NTS = true, bool NTC = true, bool LEAN = false>
 __device__ __forceinline__ EtdOps<T> etd_load(const StageArgs<T>& a, long long ubase, uint32_t off) {
   const int stage = ST >= 0 ? ST : a.stage;
   const cpx<T> zc = {(T)0, (T)0};
@@ -678,39 +721,39 @@ __device__ __forceinline__ EtdOps<T> etd_load(const StageArgs<T>& a, long long u
   // the compensated low parts exist only in the mixed (FP32) form
   constexpr bool kMixed = sizeof(T) == 4;
   if (stage <= 2) {
-    const cpx<T> s0 = ld_pol<NTS>(a.sol + ubase + off);
+    const cpx<T> s0 = ld_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off));
     o.sr = (double)s0.re;
     o.si = (double)s0.im;
     if (kMixed && a.sol_lo) {
-      const cpx<T> lo = ld_pol<NTS>(a.sol_lo + ubase + off);
+      const cpx<T> lo = ld_pol<NTS>(lane_at<LEAN>(a.sol_lo + ubase, off));
       o.sr += (double)lo.re;
       o.si += (double)lo.im;
     }
-    o.e2 = ld_pol<NTC>(a.E2 + ubase + off);
-    o.z = ld_pol<NTC>(a.zeta + ubase + off);
+    o.e2 = ld_pol<NTC>(lane_at<LEAN>(a.E2 + ubase, off));
+    o.z = ld_pol<NTC>(lane_at<LEAN>(a.zeta + ubase, off));
     if (stage == 2) {
-      o.s1 = ld_pol<NTS>(a.stg + ubase + off);
-      o.n1 = ld_pol<NTS>(a.n1 + ubase + off);
-      o.n2 = ld_pol<NTS>(a.n2 + ubase + off);
-      o.e = ld_pol<NTC>(a.E + ubase + off);
-      o.al = ld_pol<NTC>(a.alpha + ubase + off);
-      o.be = ld_pol<NTC>(a.beta + ubase + off);
+      o.s1 = ld_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off));
+      o.n1 = ld_pol<NTS>(lane_at<LEAN>(a.n1 + ubase, off));
+      o.n2 = ld_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off));
+      o.e = ld_pol<NTC>(lane_at<LEAN>(a.E + ubase, off));
+      o.al = ld_pol<NTC>(lane_at<LEAN>(a.alpha + ubase, off));
+      o.be = ld_pol<NTC>(lane_at<LEAN>(a.beta + ubase, off));
     }
   } else {
-    const cpx<T> ac = ld_pol<NTS>(a.acc + ubase + off);
+    const cpx<T> ac = ld_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off));
     o.sr = (double)ac.re;
     o.si = (double)ac.im;
     if (kMixed && a.sol_lo) {
-      const cpx<T> al = ld_pol<NTS>(a.n2 + ubase + off);   // the low part of acc
+      const cpx<T> al = ld_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off));   // the low part of acc
       o.sr += (double)al.re;
       o.si += (double)al.im;
     }
-    o.g = ld_pol<NTC>(a.gam + ubase + off);
+    o.g = ld_pol<NTC>(lane_at<LEAN>(a.gam + ubase, off));
   }
   return o;
 }
 
-template <typename T, int ST = -1, bool NTS = true>
+template <typename T, int ST = -1, bool NTS = true, bool LEAN = false>
 __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ubase, uint32_t off,
                                              int ikx, int iky, int ikz, cpx<T> N,
                                              const EtdOps<T>& o, bool store = true) {
@@ -721,11 +764,11 @@ __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ub
     const cpx<T> v = {(T)(o.e2 * o.sr + o.z * nre), (T)(o.e2 * o.si + o.z * nim)};
     if (store) {
       if (stage == 0) {
-        st_pol<NTS>(a.stg + ubase + off, v);
-        st_pol<NTS>(a.n1 + ubase + off, N);
+        st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), v);
+        st_pol<NTS>(lane_at<LEAN>(a.n1 + ubase, off), N);
       } else {
-        st_pol<NTS>(a.stg2 + ubase + off, v);
-        st_pol<NTS>(a.n2 + ubase + off, N);
+        st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
+        st_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off), N);
       }
     }
     return v;
@@ -737,10 +780,10 @@ __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ub
     const double ai = o.e * o.si + o.al * (double)o.n1.im + be2 * ((double)o.n2.im + nim);
     const cpx<T> hi = {(T)ar, (T)ai};
     if (store) {
-      st_pol<NTS>(a.stg2 + ubase + off, v);
-      st_pol<NTS>(a.acc + ubase + off, hi);
+      st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
+      st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), hi);
       if (kMixed && a.sol_lo)   // the low part of acc
-        st_pol<NTS>(a.n2 + ubase + off, {(T)(ar - (double)hi.re), (T)(ai - (double)hi.im)});
+        st_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off), {(T)(ar - (double)hi.re), (T)(ai - (double)hi.im)});
     }
     return v;
   } else {
@@ -752,9 +795,9 @@ __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ub
     }
     const cpx<T> hi = {(T)sr, (T)si};
     if (store) {
-      st_pol<NTS>(a.sol + ubase + off, hi);
+      st_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off), hi);
       if (kMixed && a.sol_lo)
-        st_pol<NTS>(a.sol_lo + ubase + off, {(T)(sr - (double)hi.re), (T)(si - (double)hi.im)});
+        st_pol<NTS>(lane_at<LEAN>(a.sol_lo + ubase, off), {(T)(sr - (double)hi.re), (T)(si - (double)hi.im)});
     }
     return hi;
   }

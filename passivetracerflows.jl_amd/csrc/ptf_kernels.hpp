@@ -179,6 +179,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, TX * (N / R)),
 void col_kernel(ColArgs<T> a) {
   static_assert(epf_ok<MODE, EPF>(), "stage kernels take an epilogue family, others none");
   constexpr int P = N / R;
+  constexpr bool kLean = fft_lean<T, R, OCC>();
   // Non-temporal loads (and state stores) only where a block covers whole 128-byte lines
   // of a field: along the bricked axis a column's run is the 8 planes of a brick, so a
   // block reads TX * 8 consecutive elements; the columns of the 3D y pass are contiguous
@@ -216,19 +217,24 @@ void col_kernel(ColArgs<T> a) {
   // the line transform in direction D with this block's twiddle source
   auto fft = [&](auto dir_c, cpx<T>(&x)[R]) {
     constexpr int D = decltype(dir_c)::value;
-    if constexpr (col_tw_lds<N, R>()) line_fft<T, N, R, D, Lay, kTwh>(x, lds, lay, c, j, twl, 1, wave);
-    else line_fft<T, N, R, D, Lay>(x, lds, lay, c, j, a.tw, a.twstride, wave);
+    if constexpr (col_tw_lds<N, R>()) line_fft<T, N, R, D, Lay, kTwh, kLean>(x, lds, lay, c, j, twl, 1, wave);
+    else line_fft<T, N, R, D, Lay, false, kLean>(x, lds, lay, c, j, a.tw, a.twstride, wave);
   };
   int bx, by, member;
   xcd_remap(bx, by, member);
   const int kx = bx * TX + c;
   const bool valid = kx < a.ncols;
   const int kxc = valid ? kx : a.ncols - 1;   // invalid lanes load a valid column, store nothing
-  // block-uniform base (SGPRs) + 32-bit lane offsets
-  const long long ubase = (long long)member * a.mstride + (long long)by * a.ostride;
+  // Element j + q P of the line: a block-uniform base (SGPRs) plus a 32-bit lane offset.  In
+  // the lean builds the base includes q's planes and the wavefront's first plane jh0 (jh never
+  // falls below its first lane's), so that one lane offset serves all q; the rest jh - jh0 is at
+  // most 7 on bricked lines and 63 / TX on plain ones, so its bytes stay below 4 GiB.
+  const int jh0 = kLean ? __builtin_amdgcn_readfirstlane(jh) : 0;
+  const long long ubase0 = (long long)member * a.mstride + (long long)by * a.ostride + jh0 * a.stride;
   const uint32_t s = (uint32_t)a.stride;
+  auto ub = [&](int q) -> long long { return kLean ? ubase0 + (long long)(q * (P >> lb)) * a.stride : ubase0; };
   auto off = [&](int q) -> uint32_t {
-    return ((uint32_t)kxc << lb) + (uint32_t)rb + (uint32_t)(jh + q * (P >> lb)) * s;
+    return ((uint32_t)kxc << lb) + (uint32_t)rb + (uint32_t)(jh - jh0 + (kLean ? 0 : q * (P >> lb))) * s;
   };
   // wavenumber indices of this lane's column (3D y pass over folded columns)
   const int ikx_col = kx >> a.lbc;
@@ -236,16 +242,14 @@ void col_kernel(ColArgs<T> a) {
 
   cpx<T> v[R];
   if constexpr (MODE == COL_FLOWSYN) {
-    const cpx<double>* ps = a.psih0 + ubase;
-    const double* om = a.omega + ubase;
     // out1 = IFFT_y(i kr psi(t)) first, then out0 = IFFT_y(-i l psi(t)); psi(t) is formed
     // once (one read of psih0 and omega), both inputs at once
     cpx<T> w[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int iy = j + q * P;
-      const cpx<double> p0 = ps[off(q)];
-      const double ph = -om[off(q)] * a.t;
+      const cpx<double> p0 = *lane_at<kLean>(a.psih0 + ub(q), off(q));
+      const double ph = -*lane_at<kLean>(a.omega + ub(q), off(q)) * a.t;
       double sn, cs;
       sincos(ph, &sn, &cs);
       const cpx<double> p = {p0.re * cs - p0.im * sn, p0.re * sn + p0.im * cs};
@@ -261,28 +265,27 @@ void col_kernel(ColArgs<T> a) {
         for (int q = 0; q < R; ++q) v[q] = w[q];
       }
       fft(std::integral_constant<int, 1>{}, v);
-      cpx<T>* o = (pass == 0 ? a.out1 : a.out0) + ubase;
+      cpx<T>* o = pass == 0 ? a.out1 : a.out0;
       if (valid) {
 #pragma unroll
-        for (int q = 0; q < R; ++q) o[off(q)] = v[q];
+        for (int q = 0; q < R; ++q) *lane_at<kLean>(o + ub(q), off(q)) = v[q];
       }
     }
     return;
   } else {
-    const cpx<T>* in0 = a.in0 + ubase;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       // the 3D y-inverse pass reads its inputs once: non-temporal loads there
-      if constexpr (MODE == COL_D2) v[q] = ld_pol<kNtS>(in0 + off(q));
-      else v[q] = in0[off(q)];
+      if constexpr (MODE == COL_D2) v[q] = ld_pol<kNtS>(lane_at<kLean>(a.in0 + ub(q), off(q)));
+      else v[q] = *lane_at<kLean>(a.in0 + ub(q), off(q));
     }
 
     if constexpr (MODE == COL_PLAIN) {
       fft(std::integral_constant<int, DIR>{}, v);
-      cpx<T>* o = a.out0 + ubase;
+      cpx<T>* o = a.out0;
       if (valid) {
 #pragma unroll
-        for (int q = 0; q < R; ++q) o[off(q)] = v[q];
+        for (int q = 0; q < R; ++q) *lane_at<kLean>(o + ub(q), off(q)) = v[q];
       }
     } else if constexpr (MODE == COL_D1 || MODE == COL_D2) {
       // The derivative is transformed and stored first, because out0 may alias in0
@@ -295,9 +298,8 @@ void col_kernel(ColArgs<T> a) {
 #pragma unroll
       for (int q = 0; q < R; ++q) u[q] = v[q];
       if constexpr (kKeep && MODE == COL_D2) {
-        const cpx<T>* in1 = a.in1 + ubase;
 #pragma unroll
-        for (int q = 0; q < R; ++q) p2[q] = ld_pol<kNtS>(in1 + off(q));
+        for (int q = 0; q < R; ++q) p2[q] = ld_pol<kNtS>(lane_at<kLean>(a.in1 + ub(q), off(q)));
       }
 #pragma unroll
       for (int q = 0; q < R; ++q) {
@@ -306,34 +308,33 @@ void col_kernel(ColArgs<T> a) {
       }
       fft(std::integral_constant<int, 1>{}, v);
       {
-        cpx<T>* o = a.out1 + ubase;
+        cpx<T>* o = a.out1;
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) o[off(q)] = v[q];
+          for (int q = 0; q < R; ++q) *lane_at<kLean>(o + ub(q), off(q)) = v[q];
         }
       }
 #pragma unroll
       for (int q = 0; q < R; ++q) v[q] = u[q];
       fft(std::integral_constant<int, 1>{}, v);
       {
-        cpx<T>* o = a.out0 + ubase;
+        cpx<T>* o = a.out0;
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) o[off(q)] = v[q];
+          for (int q = 0; q < R; ++q) *lane_at<kLean>(o + ub(q), off(q)) = v[q];
         }
       }
       if constexpr (MODE == COL_D2) {
-        const cpx<T>* in1 = a.in1 + ubase;
 #pragma unroll
         for (int q = 0; q < R; ++q) {
           if constexpr (kKeep) v[q] = p2[q];
-          else v[q] = ld_pol<kNtS>(in1 + off(q));
+          else v[q] = ld_pol<kNtS>(lane_at<kLean>(a.in1 + ub(q), off(q)));
         }
         fft(std::integral_constant<int, 1>{}, v);
-        cpx<T>* o = a.out2 + ubase;
+        cpx<T>* o = a.out2;
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) o[off(q)] = v[q];
+          for (int q = 0; q < R; ++q) *lane_at<kLean>(o + ub(q), off(q)) = v[q];
         }
       }
     } else if constexpr (MODE == COL_STAGE || MODE == COL_STAGE_D1) {
@@ -359,7 +360,7 @@ void col_kernel(ColArgs<T> a) {
           stage_dispatch([&](auto stc) {
             constexpr int ST = decltype(stc)::value;
 #pragma unroll
-            for (int q = 0; q < R; ++q) ops[q] = rk4_load<T, ST, kNtS>(a.st, ubase, off(q));
+            for (int q = 0; q < R; ++q) ops[q] = rk4_load<T, ST, kNtS, kLean>(a.st, ub(q), off(q));
           });
         }
       }
@@ -375,7 +376,7 @@ void col_kernel(ColArgs<T> a) {
             Rk4Ops<T> o[kChunk];
             if constexpr (!kPre) {
 #pragma unroll
-              for (int i = 0; i < kChunk; ++i) o[i] = rk4_load<T, ST, kNtS>(a.st, ubase, off(q0 + i));
+              for (int i = 0; i < kChunk; ++i) o[i] = rk4_load<T, ST, kNtS, kLean>(a.st, ub(q0 + i), off(q0 + i));
             }
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
@@ -386,7 +387,7 @@ void col_kernel(ColArgs<T> a) {
               Rk4Ops<T> oq;
               if constexpr (kPre) oq = ops[q];
               else oq = o[i];
-              v[q] = rk4_finish<T, ST, kNtS>(a.st, ubase, off(q), opm, ikx_col, iky, ikz, v[q], oq, valid);
+              v[q] = rk4_finish<T, ST, kNtS, kLean>(a.st, ub(q), off(q), opm, ikx_col, iky, ikz, v[q], oq, valid);
             }
           }
         });
@@ -398,14 +399,14 @@ void col_kernel(ColArgs<T> a) {
           for (int q0 = 0; q0 < R; q0 += kChunk) {
             EtdOps<T> o[kChunk];
 #pragma unroll
-            for (int i = 0; i < kChunk; ++i) o[i] = etd_load<T, ST, kNtS, kNtC>(a.st, ubase, off(q0 + i));
+            for (int i = 0; i < kChunk; ++i) o[i] = etd_load<T, ST, kNtS, kNtC, kLean>(a.st, ub(q0 + i), off(q0 + i));
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
               const int q = q0 + i;
               const int ia = j + q * P;
               const int iky = a.axis == 2 ? by : ia;
               const int ikz = a.axis == 2 ? ia : iklast_col;
-              v[q] = etd_finish<T, ST, kNtS>(a.st, ubase, off(q), ikx_col, iky, ikz, v[q], o[i], valid);
+              v[q] = etd_finish<T, ST, kNtS, kLean>(a.st, ub(q), off(q), ikx_col, iky, ikz, v[q], o[i], valid);
             }
           }
         });
@@ -413,7 +414,7 @@ void col_kernel(ColArgs<T> a) {
         // plain store of the transformed line (calcN! without a stage update)
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) (a.out0 + ubase)[off(q)] = v[q];
+          for (int q = 0; q < R; ++q) *lane_at<kLean>(a.out0 + ub(q), off(q)) = v[q];
         }
       }
       if constexpr (MODE == COL_STAGE_D1) {
@@ -436,10 +437,10 @@ void col_kernel(ColArgs<T> a) {
         }
         fft(std::integral_constant<int, 1>{}, v);
         {
-          cpx<T>* op = a.out1 + ubase;
+          cpx<T>* op = a.out1;
           if (valid) {
 #pragma unroll
-            for (int q = 0; q < R; ++q) op[off(q)] = v[q];
+            for (int q = 0; q < R; ++q) *lane_at<kLean>(op + ub(q), off(q)) = v[q];
           }
         }
 #pragma unroll
@@ -448,10 +449,10 @@ void col_kernel(ColArgs<T> a) {
           else v[q] = w[q];
         }
         fft(std::integral_constant<int, 1>{}, v);
-        cpx<T>* op = a.out0 + ubase;
+        cpx<T>* op = a.out0;
         if (valid) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) op[off(q)] = v[q];
+          for (int q = 0; q < R; ++q) *lane_at<kLean>(op + ub(q), off(q)) = v[q];
         }
       }
     }
@@ -508,7 +509,9 @@ void col_pipe_kernel(ColArgs<T> a) {
     if constexpr (col_tw_lds<N, R>()) line_fft<T, N, R, D, Lay>(x, lds, lay, c, j, twl, 1);
     else line_fft<T, N, R, D, Lay>(x, lds, lay, c, j, a.tw, a.twstride);
   };
-  const uint32_t s = (uint32_t)a.stride;
+  // wavefront-uniform bases and one lane offset per tile (as in col_kernel)
+  const int jh0 = __builtin_amdgcn_readfirstlane(jh);
+  const long long qstep = (long long)(P >> lb) * a.stride;
 
   // this block's tiles: XCD range [lo, hi), visited with stride = blocks on the XCD (with
   // fewer than 8 blocks, each block is its own range)
@@ -524,6 +527,7 @@ void col_pipe_kernel(ColArgs<T> a) {
     int bx, by, member, kx, kxc;
     bool valid;
     long long ubase;
+    uint32_t loff;
   };
   auto tile_at = [&](unsigned L) {
     Tile u;
@@ -533,16 +537,14 @@ void col_pipe_kernel(ColArgs<T> a) {
     u.kx = u.bx * TX + c;
     u.valid = u.kx < a.ncols;
     u.kxc = u.valid ? u.kx : a.ncols - 1;
-    u.ubase = (long long)u.member * a.mstride + (long long)u.by * a.ostride;
+    u.ubase = (long long)u.member * a.mstride + (long long)u.by * a.ostride + jh0 * a.stride;
+    u.loff = ((uint32_t)u.kxc << lb) + (uint32_t)rb + (uint32_t)(jh - jh0) * (uint32_t)a.stride;
     return u;
   };
-  auto off = [&](const Tile& u, int q) -> uint32_t {
-    return ((uint32_t)u.kxc << lb) + (uint32_t)rb + (uint32_t)(jh + q * (P >> lb)) * s;
-  };
+  auto ub = [&](const Tile& u, int q) -> long long { return u.ubase + q * qstep; };
   auto load_line = [&](const Tile& u, cpx<T>(&v)[R]) {
-    const cpx<T>* in0 = a.in0 + u.ubase;
 #pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = in0[off(u, q)];
+    for (int q = 0; q < R; ++q) v[q] = *lane_at(a.in0 + ub(u, q), u.loff);
   };
 
   const bool rk4 = EPF == EPF_RK4 || (EPF == EPF_ANY && a.st.kind == EPI_RK4);
@@ -567,17 +569,15 @@ void col_pipe_kernel(ColArgs<T> a) {
     }
     fft(std::integral_constant<int, 1>{}, v);
     if (u.valid) {
-      cpx<T>* o1 = a.out1 + u.ubase;
 #pragma unroll
-      for (int q = 0; q < R; ++q) o1[off(u, q)] = v[q];
+      for (int q = 0; q < R; ++q) *lane_at(a.out1 + ub(u, q), u.loff) = v[q];
     }
 #pragma unroll
     for (int q = 0; q < R; ++q) v[q] = keep[q];
     fft(std::integral_constant<int, 1>{}, v);
     if (u.valid) {
-      cpx<T>* o0 = a.out0 + u.ubase;
 #pragma unroll
-      for (int q = 0; q < R; ++q) o0[off(u, q)] = v[q];
+      for (int q = 0; q < R; ++q) *lane_at(a.out0 + ub(u, q), u.loff) = v[q];
     }
   };
 
@@ -591,7 +591,7 @@ void col_pipe_kernel(ColArgs<T> a) {
       Rk4Ops<T> ops[R];
       load_line(cur, v);
 #pragma unroll
-      for (int q = 0; q < R; ++q) ops[q] = rk4_load<T, ST, kNtS>(a.st, cur.ubase, off(cur, q));
+      for (int q = 0; q < R; ++q) ops[q] = rk4_load<T, ST, kNtS>(a.st, ub(cur, q), cur.loff);
       for (;;) {
         const unsigned Ln = L + per_xcd_blocks;
         const bool more = Ln < hi;
@@ -603,7 +603,7 @@ void col_pipe_kernel(ColArgs<T> a) {
           nxt = tile_at(Ln);
           load_line(nxt, vn);
 #pragma unroll
-          for (int q = 0; q < R; ++q) opsn[q] = rk4_load<T, ST, kNtS>(a.st, nxt.ubase, off(nxt, q));
+          for (int q = 0; q < R; ++q) opsn[q] = rk4_load<T, ST, kNtS>(a.st, ub(nxt, q), nxt.loff);
         }
         fft(std::integral_constant<int, -1>{}, v);
         const OpParams opm = a.st.op[cur.member];
@@ -614,7 +614,7 @@ void col_pipe_kernel(ColArgs<T> a) {
           const int ia = j + q * P;
           const int iky = a.axis == 2 ? cur.by : ia;
           const int ikz = a.axis == 2 ? ia : iklast;
-          v[q] = rk4_finish<T, ST, kNtS>(a.st, cur.ubase, off(cur, q), opm, ikx, iky, ikz, v[q], ops[q],
+          v[q] = rk4_finish<T, ST, kNtS>(a.st, ub(cur, q), cur.loff, opm, ikx, iky, ikz, v[q], ops[q],
                                    cur.valid);
         }
         next_stage_inverse(cur, v);
@@ -653,14 +653,14 @@ void col_pipe_kernel(ColArgs<T> a) {
         for (int q0 = 0; q0 < R; q0 += kChunk) {
           EtdOps<T> o[kChunk];
 #pragma unroll
-          for (int i = 0; i < kChunk; ++i) o[i] = etd_load<T, ST, kNtS, kNtC>(a.st, cur.ubase, off(cur, q0 + i));
+          for (int i = 0; i < kChunk; ++i) o[i] = etd_load<T, ST, kNtS, kNtC>(a.st, ub(cur, q0 + i), cur.loff);
 #pragma unroll
           for (int i = 0; i < kChunk; ++i) {
             const int q = q0 + i;
             const int ia = j + q * P;
             const int iky = a.axis == 2 ? cur.by : ia;
             const int ikz = a.axis == 2 ? ia : iklast;
-            v[q] = etd_finish<T, ST, kNtS>(a.st, cur.ubase, off(cur, q), ikx, iky, ikz, v[q], o[i], cur.valid);
+            v[q] = etd_finish<T, ST, kNtS>(a.st, ub(cur, q), cur.loff, ikx, iky, ikz, v[q], o[i], cur.valid);
           }
         }
         next_stage_inverse(cur, v);
@@ -751,24 +751,25 @@ __device__ __forceinline__ void stage_row_pairs(const cpx<T> (&x)[R], cpx<T> las
   for (int q = 0; q < R; ++q) xm[q] = lds[lay.idx(c, M - (j + q * P))];
 }
 
-// Row element k is row[k << lb] (brick layout; lb = 0 for contiguous rows).  The x
-// pass reads each spectral row once per stage: non-temporal loads (NT), where the
-// block holds whole bricks of rows (see row_nt).
-template <typename T, int M, int R, bool NT = true>
-__device__ __forceinline__ void load_row(const cpx<T>* __restrict__ row, cpx<T> (&x)[R],
+// Row element k sits at k << lb from the row's start (brick layout; lb = 0 for contiguous
+// rows): base is block-uniform, off the lane's offset to its element j.  The x pass reads each
+// spectral row once per stage: non-temporal loads (NT), where the block holds whole bricks of
+// rows (see row_nt).
+template <typename T, int M, int R, bool NT, bool LEAN>
+__device__ __forceinline__ void load_row(const cpx<T>* base, uint32_t off, cpx<T> (&x)[R],
                                          cpx<T>& last, int j, int lb) {
   constexpr int P = M / R;
 #pragma unroll
-  for (int q = 0; q < R; ++q) x[q] = ld_pol<NT>(row + ((uint32_t)(j + q * P) << lb));
-  if (j == 0) last = ld_pol<NT>(row + ((uint32_t)M << lb));
+  for (int q = 0; q < R; ++q) x[q] = ld_pol<NT>(lane_at<LEAN>(base + ((uint32_t)(q * P) << lb), off));
+  if (j == 0) last = ld_pol<NT>(lane_at<LEAN>(base + ((uint32_t)M << lb), off));
 }
 
-template <typename T, int M, int R, class Lay, bool NT = true>
-__device__ __forceinline__ void load_row_pairs(const cpx<T>* __restrict__ row, cpx<T> (&x)[R],
+template <typename T, int M, int R, class Lay, bool NT, bool LEAN>
+__device__ __forceinline__ void load_row_pairs(const cpx<T>* base, uint32_t off, cpx<T> (&x)[R],
                                                cpx<T> (&xm)[R], cpx<T>* lds, const Lay& lay, int c,
                                                int j, int lb) {
   cpx<T> last = {(T)0, (T)0};
-  load_row<T, M, R, NT>(row, x, last, j, lb);
+  load_row<T, M, R, NT, LEAN>(base, off, x, last, j, lb);
   stage_row_pairs<T, M, R, Lay>(x, last, xm, lds, lay, c, j);
 }
 
@@ -813,6 +814,7 @@ void row_kernel(RowArgs<T> a) {
   constexpr int M = NX / 2;
   constexpr int NXH = M + 1;
   constexpr int P = M / R;
+  constexpr bool kLean = fft_lean<T, R, OCC>();
   // LDS rows hold M + 1 entries (X[M] while staging a row).  Contiguous rows
   // (lanes walk a row) are stored row-major; bricked rows (lanes walk the rows
   // of a brick first) element-major, so a wavefront's accesses stay contiguous.
@@ -850,27 +852,29 @@ void row_kernel(RowArgs<T> a) {
   // block-uniform bases + 32-bit lane offsets
   const long long sub = (long long)member * a.smstride + brick_row_base(row0, lb, NXH);
   const long long pub = (long long)member * a.pmstride + 2 * brick_row_base(row0, lb, M);
-  const uint32_t so = ((uint32_t)gc * NXH << lb) + rb;           // spectral element 0 (loads)
-  const uint32_t so_st = ((uint32_t)g * NXH << lb) + rb;         // (stores)
-  const uint32_t po = ((uint32_t)gc * M << lb) + rb;             // physical pair 0 (loads)
-  const uint32_t po_st = ((uint32_t)g * M << lb) + rb;           // (stores)
+  const uint32_t so = ((uint32_t)gc * NXH << lb) + rb + ((uint32_t)j << lb);     // spectral element j (loads)
+  const uint32_t so_st = ((uint32_t)g * NXH << lb) + rb + ((uint32_t)j << lb);   // (stores)
+  const uint32_t po = ((uint32_t)gc * M << lb) + rb + ((uint32_t)j << lb);       // physical pair j (loads)
+  const uint32_t po_st = ((uint32_t)g * M << lb) + rb + ((uint32_t)j << lb);     // (stores)
+  // element j + q P from element j (uniform)
+  auto qoff = [&](int q) -> uint32_t { return (uint32_t)(q * P) << lb; };
   const cpx<T> zero = {(T)0, (T)0};
 
   if constexpr (MODE == ROW_C2R) {
     cpx<T> z[R], zm[R];
     const T s = (T)a.scale;
-    load_row_pairs<T, M, R, Lay, row_nt<NL>()>(a.in[0] + sub + so, z, zm, lds, lay, c, j, lb);
+    load_row_pairs<T, M, R, Lay, row_nt<NL>(), kLean>(a.in[0] + sub, so, z, zm, lds, lay, c, j, lb);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int k = j + q * P;
       z[q] = c2r_pre(z[q], zm[q], (row_tw_lds<NX>() ? twl[k] : a.tw[k * a.twstride]), s, k == 0);
     }
-    if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh>(z, lds, lay, c, j, twl, 2);
-    else line_fft<T, M, R, +1, Lay>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
+    if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh, kLean>(z, lds, lay, c, j, twl, 2);
+    else line_fft<T, M, R, +1, Lay, false, kLean>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
     if (valid) {
       cpx<T>* out = reinterpret_cast<cpx<T>*>(a.rout + pub);
 #pragma unroll
-      for (int q = 0; q < R; ++q) out[po_st + ((uint32_t)(j + q * P) << lb)] = z[q];
+      for (int q = 0; q < R; ++q) *lane_at<kLean>(out + qoff(q), po_st) = z[q];
     }
     return;
   } else {
@@ -878,7 +882,7 @@ void row_kernel(RowArgs<T> a) {
     if constexpr (MODE == ROW_R2C) {
       const cpx<T>* rin = reinterpret_cast<const cpx<T>*>(a.rin + pub);
 #pragma unroll
-      for (int q = 0; q < R; ++q) f[q] = rin[po + ((uint32_t)(j + q * P) << lb)];
+      for (int q = 0; q < R; ++q) f[q] = *lane_at<kLean>(rin + qoff(q), po);
     } else {
       // ROW_ADV: f = ((-u cx) - v cy) - w cz, cx = C2R(i kr Y0), cy = C2R(Y1), cz = C2R(Y2)
       const T s = (T)a.scale;
@@ -891,7 +895,7 @@ void row_kernel(RowArgs<T> a) {
       constexpr bool kPre = sizeof(T) == 4 || R <= 4;
       cpx<T> nxt[kPre ? R : 1];
       cpx<T> nlast = zero;
-      if constexpr (kPre) load_row<T, M, R, row_nt<NL>()>(a.in[0] + sub + so, nxt, nlast, j, lb);
+      if constexpr (kPre) load_row<T, M, R, row_nt<NL>(), kLean>(a.in[0] + sub, so, nxt, nlast, j, lb);
 #pragma unroll 1
       for (int d = 0; d < NIN; ++d) {
         cpx<T> z[R], zm[R];
@@ -899,15 +903,15 @@ void row_kernel(RowArgs<T> a) {
 #pragma unroll
           for (int q = 0; q < R; ++q) z[q] = nxt[q];
           stage_row_pairs<T, M, R, Lay>(z, nlast, zm, lds, lay, c, j);
-          if (d + 1 < NIN) load_row<T, M, R, row_nt<NL>()>(in_at(d + 1) + sub + so, nxt, nlast, j, lb);
+          if (d + 1 < NIN) load_row<T, M, R, row_nt<NL>(), kLean>(uniform_ptr(in_at(d + 1) + sub), so, nxt, nlast, j, lb);
         } else {
-          load_row_pairs<T, M, R, Lay, row_nt<NL>()>(in_at(d) + sub + so, z, zm, lds, lay, c, j, lb);
+          load_row_pairs<T, M, R, Lay, row_nt<NL>(), kLean>(uniform_ptr(in_at(d) + sub), so, z, zm, lds, lay, c, j, lb);
         }
-        const cpx<T>* fl = reinterpret_cast<const cpx<T>*>(flow_at(d) + pub);
+        const cpx<T>* fl = uniform_ptr(reinterpret_cast<const cpx<T>*>(flow_at(d) + pub));
         cpx<T> fv[kPre ? R : 1];
         if constexpr (kPre) {
 #pragma unroll
-          for (int q = 0; q < R; ++q) fv[q] = ld_pol<row_nt<NL>()>(fl + po + ((uint32_t)(j + q * P) << lb));
+          for (int q = 0; q < R; ++q) fv[q] = ld_pol<row_nt<NL>()>(lane_at<kLean>(fl + qoff(q), po));
         }
 #pragma unroll
         for (int q = 0; q < R; ++q) {
@@ -920,13 +924,13 @@ void row_kernel(RowArgs<T> a) {
           }
           z[q] = c2r_pre(Xk, Xm, (row_tw_lds<NX>() ? twl[k] : a.tw[k * a.twstride]), s, k == 0);
         }
-        if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh>(z, lds, lay, c, j, twl, 2);
-        else line_fft<T, M, R, +1, Lay>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
+        if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh, kLean>(z, lds, lay, c, j, twl, 2);
+        else line_fft<T, M, R, +1, Lay, false, kLean>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
 #pragma unroll
         for (int q = 0; q < R; ++q) {
           cpx<T> uu;
           if constexpr (kPre) uu = fv[q];
-          else uu = ld_pol<row_nt<NL>()>(fl + po + ((uint32_t)(j + q * P) << lb));
+          else uu = ld_pol<row_nt<NL>()>(lane_at<kLean>(fl + qoff(q), po));
           if (d == 0) {
             f[q] = {-uu.re * z[q].re, -uu.im * z[q].im};
           } else {
@@ -936,8 +940,8 @@ void row_kernel(RowArgs<T> a) {
       }
     }
     // forward half-length FFT of f[2m] + i f[2m+1]
-    if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, -1, Lay, kTwh>(f, lds, lay, c, j, twl, 2);
-    else line_fft<T, M, R, -1, Lay>(f, lds, lay, c, j, a.tw, 2 * a.twstride);
+    if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, -1, Lay, kTwh, kLean>(f, lds, lay, c, j, twl, 2);
+    else line_fft<T, M, R, -1, Lay, false, kLean>(f, lds, lay, c, j, a.tw, 2 * a.twstride);
     // exchange Z[M-k] through LDS
     __syncthreads();
 #pragma unroll
@@ -965,15 +969,15 @@ void row_kernel(RowArgs<T> a) {
         bool epi = false;
         if constexpr (kEpi) epi = a.st.kind != EPI_STORE;
         if constexpr (kEpi) {
-          if (epi) (void)stage_epilogue(a.st, sub, so_st + ((uint32_t)k << lb), member, k, iky, ikz, X);
+          if (epi) (void)stage_epilogue(a.st, sub + qoff(q), so_st, member, k, iky, ikz, X);
         }
-        if (!epi) (a.out + sub)[so_st + ((uint32_t)k << lb)] = X;
+        if (!epi) *lane_at<kLean>(a.out + sub + qoff(q), so_st) = X;
         if (k == 0) {
           const cpx<T> XM = {f[q].re - f[q].im, (T)0};
           if constexpr (kEpi) {
-            if (epi) (void)stage_epilogue(a.st, sub, so_st + ((uint32_t)M << lb), member, M, iky, ikz, XM);
+            if (epi) (void)stage_epilogue(a.st, sub + ((uint32_t)M << lb), so_st, member, M, iky, ikz, XM);
           }
-          if (!epi) (a.out + sub)[so_st + ((uint32_t)M << lb)] = XM;
+          if (!epi) *lane_at<kLean>(a.out + sub + ((uint32_t)M << lb), so_st) = XM;
         }
       }
     }
@@ -1005,6 +1009,7 @@ void row_adv_par_kernel(RowArgs<T> a) {
   constexpr int M = NX / 2;
   constexpr int NXH = M + 1;
   constexpr int P = M / R;
+  constexpr bool kLean = fft_lean<T, R, OCC>();
   constexpr int G = NL * P;   // threads per group
   static_assert(G % 64 == 0, "a group must be whole wavefronts");
   static_assert(NIN >= 2 && NIN <= 3, "two or three inputs");
@@ -1017,7 +1022,7 @@ void row_adv_par_kernel(RowArgs<T> a) {
     // every group fills (before any group ends); read after the first row exchange
     for (int i = (int)threadIdx.x; i < row_tw_elems<T, NX>(); i += (int)blockDim.x) twl[i] = a.tw[i * a.twstride];
   }
-  const int grp = (int)threadIdx.x / G;   // uniform over a wavefront
+  const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / G);   // uniform over a wavefront
   const int t = (int)threadIdx.x - grp * G;
   cpx<T>* lds = lds_all + grp * (NL * (M + 1));
   // lane and block mapping as in row_kernel
@@ -1040,19 +1045,20 @@ void row_adv_par_kernel(RowArgs<T> a) {
   const int gc = valid ? g : (g < gmax ? g : gmax);
   const long long sub = (long long)member * a.smstride + brick_row_base(row0, lb, NXH);
   const long long pub = (long long)member * a.pmstride + 2 * brick_row_base(row0, lb, M);
-  const uint32_t so = ((uint32_t)gc * NXH << lb) + rb;
-  const uint32_t so_st = ((uint32_t)g * NXH << lb) + rb;
-  const uint32_t po = ((uint32_t)gc * M << lb) + rb;
+  const uint32_t so = ((uint32_t)gc * NXH << lb) + rb + ((uint32_t)j << lb);
+  const uint32_t so_st = ((uint32_t)g * NXH << lb) + rb + ((uint32_t)j << lb);
+  const uint32_t po = ((uint32_t)gc * M << lb) + rb + ((uint32_t)j << lb);
+  auto qoff = [&](int q) -> uint32_t { return (uint32_t)(q * P) << lb; };
   const T s = (T)a.scale;
   // select, not a.in[grp]: a runtime index into the by-value arguments would go to scratch
   const cpx<T>* in = grp == 0 ? a.in[0] : (grp == 1 ? a.in[1] : a.in[2]);
   const T* flp = grp == 0 ? a.flow[0] : (grp == 1 ? a.flow[1] : a.flow[2]);
   cpx<T> z[R], last = {(T)0, (T)0};
-  load_row<T, M, R, row_nt<NL>()>(in + sub + so, z, last, j, lb);
-  const cpx<T>* fl = reinterpret_cast<const cpx<T>*>(flp + pub);
+  load_row<T, M, R, row_nt<NL>(), kLean>(uniform_ptr(in + sub), so, z, last, j, lb);
+  const cpx<T>* fl = uniform_ptr(reinterpret_cast<const cpx<T>*>(flp + pub));
   cpx<T> fv[R];
 #pragma unroll
-  for (int q = 0; q < R; ++q) fv[q] = ld_pol<row_nt<NL>()>(fl + po + ((uint32_t)(j + q * P) << lb));
+  for (int q = 0; q < R; ++q) fv[q] = ld_pol<row_nt<NL>()>(lane_at<kLean>(fl + qoff(q), po));
   cpx<T> zm[R];
   stage_row_pairs<T, M, R, Lay>(z, last, zm, lds, lay, c, j);
 #pragma unroll
@@ -1066,8 +1072,8 @@ void row_adv_par_kernel(RowArgs<T> a) {
     }
     z[q] = c2r_pre(Xk, Xm, (row_tw_lds<NX>() ? twl[k] : a.tw[k * a.twstride]), s, k == 0);
   }
-  if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh>(z, lds, lay, c, j, twl, 2);
-  else line_fft<T, M, R, +1, Lay>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
+  if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, +1, Lay, kTwh, kLean>(z, lds, lay, c, j, twl, 2);
+  else line_fft<T, M, R, +1, Lay, false, kLean>(z, lds, lay, c, j, a.tw, 2 * a.twstride);
   cpx<T> f[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) f[q] = {fv[q].re * z[q].re, fv[q].im * z[q].im};
@@ -1096,8 +1102,8 @@ void row_adv_par_kernel(RowArgs<T> a) {
     f[q] = v;
   }
   // forward half-length FFT of f[2m] + i f[2m+1] (the other groups match its barriers)
-  if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, -1, Lay, kTwh>(f, lds, lay, c, j, twl, 2);
-  else line_fft<T, M, R, -1, Lay>(f, lds, lay, c, j, a.tw, 2 * a.twstride);
+  if constexpr (row_tw_lds<NX>()) line_fft<T, M, R, -1, Lay, kTwh, kLean>(f, lds, lay, c, j, twl, 2);
+  else line_fft<T, M, R, -1, Lay, false, kLean>(f, lds, lay, c, j, a.tw, 2 * a.twstride);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < R; ++q) lds[lay.idx(c, j + q * P)] = f[q];
@@ -1112,9 +1118,9 @@ void row_adv_par_kernel(RowArgs<T> a) {
     Xs[q] = k == 0 ? cpx<T>{f[q].re + f[q].im, (T)0} : r2c_post(f[q], Zm, w);
   }
   if (valid) {
-    if (j == 0) (a.out + sub)[so_st + ((uint32_t)M << lb)] = cpx<T>{f[0].re - f[0].im, (T)0};
+    if (j == 0) *lane_at<kLean>(a.out + sub + ((uint32_t)M << lb), so_st) = cpx<T>{f[0].re - f[0].im, (T)0};
 #pragma unroll
-    for (int q = 0; q < R; ++q) (a.out + sub)[so_st + ((uint32_t)(j + q * P) << lb)] = Xs[q];
+    for (int q = 0; q < R; ++q) *lane_at<kLean>(a.out + sub + qoff(q), so_st) = Xs[q];
   }
 }
 

@@ -1,0 +1,258 @@
+// Whole-run kernel for 1D problems.
+//
+// A 1D problem is one line: nothing but its own few KB is touched in a step, so a step is bound
+// by the latency of the stage kernels' memory round trips and launches (128 points FP64:
+// 23.6 us a step, four launches of one 64-lane block).  Here one workgroup advances a line by
+// `nsteps` whole steps in one launch: the state, the stage inputs, the operators and the flow
+// stay in registers, each thread holding elements j + q P (q < R) of the half-length line and
+// lane 0 the Nyquist element as well; LDS holds only the exchanges and the twiddle table.
+// Lines of up to 64 threads (256 points at radix 4) order their exchanges within one
+// wavefront, without workgroup barriers.  Radix 4 (6, 10, 3, 5 for the lengths that are no
+// powers of two): the fewest elements per lane, since a step is one chain of dependent
+// exchanges and the chip is idle beside it.  Measured: see the launch rule in ptf_api.hip.
+//
+// Per stage (calcN! S:695-710 for a steady 1D flow, then the stage update):
+//   N = R2C(-u C2R(i kr x))
+#pragma once
+#include "ptf_kernels.hpp"
+
+namespace ptf {
+
+template <typename T>
+struct LineArgs {
+  StageArgs<T> st;         // state, operators, stepper
+  const T* flow;           // physical u, members back to back
+  const cpx<T>* tw;        // exp(-2 pi i m / nx), m < nx
+  long long pmstride;      // physical values per member
+  double kscale_x;
+  double scale;            // C2R scale 1 / nx
+  int nsteps;
+};
+
+// One skew entry every 8 elements: a pass writes at the strides of its radix and reads at
+// stride 1, and both spread over the banks (as the column stage kernels' layout).
+struct LayLine {
+  __device__ __forceinline__ int idx(int, int i) const { return i + (i >> 3); }
+  __device__ __forceinline__ int idx_split(int, int i0, int off) const { return i0 + (i0 >> 3) + off + (off >> 3); }
+};
+
+// Elements per thread of a half-length line of M points; 0 where none is compiled.
+constexpr int line_run_e(int M) {
+  if (M < 8) return 0;
+  if ((M & (M - 1)) == 0) return M <= 2048 ? 4 : 0;
+  const int e3 = M % 2 == 0 ? 6 : 3, e5 = M % 2 == 0 ? 10 : 5;
+  if (M % 3 == 0 && M % 5 != 0 && fft_ok(M, e3) && M / e3 <= 512) return e3;
+  if (M % 5 == 0 && M % 3 != 0 && fft_ok(M, e5) && M / e5 <= 512) return e5;
+  return 0;
+}
+
+template <typename T, int NX, int R, bool ETD>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, (NX / 2) / R),
+                          amdgpu_waves_per_eu(1, ((NX / 2) / R + 255) / 256)))
+void line_run_kernel(LineArgs<T> a) {
+  constexpr int M = NX / 2;
+  constexpr int P = M / R;
+  constexpr bool kWave = P <= 64;
+  constexpr bool kMixed = sizeof(T) == 4;
+  const LayLine lay{};
+  __shared__ cpx<T> lds[M + 1 + (M >> 3)];
+  __shared__ cpx<T> twl[NX];
+  const int j = threadIdx.x;
+  const int member = blockIdx.x;
+  for (int i = j; i < NX; i += P) twl[i] = a.tw[i];
+  __syncthreads();
+  const long long ubase = (long long)member * a.st.mstride;
+  const OpParams opm = a.st.op[member];
+  const T dt = (T)a.st.dt, h2 = (T)(a.st.dt / 2);
+  const T sc = (T)a.scale;
+  const bool nyq = j == 0;   // lane 0 also holds element M, at index R
+  // wavenumber index of register e (other lanes' register R computes on zeros)
+  auto kof = [&](int e) { return e < R ? j + e * P : M; };
+
+  cpx<T> s[R + 1], lo[kMixed ? R + 1 : 1], u[R];
+  T L[ETD ? 1 : R + 1];
+  double E[ETD ? R + 1 : 1], E2[ETD ? R + 1 : 1], ze[ETD ? R + 1 : 1], al[ETD ? R + 1 : 1], be[ETD ? R + 1 : 1],
+      ga[ETD ? R + 1 : 1];
+  double fil[R + 1];
+  const cpx<T>* up = reinterpret_cast<const cpx<T>*>(a.flow + (long long)member * a.pmstride);
+#pragma unroll
+  for (int q = 0; q < R; ++q) u[q] = up[j + q * P];
+#pragma unroll
+  for (int e = 0; e <= R; ++e) {
+    const int k = kof(e);
+    const bool have = e < R || nyq;
+    s[e] = {(T)0, (T)0};
+    if (have) s[e] = a.st.sol[ubase + k];
+    if constexpr (kMixed) {
+      lo[e] = {(T)0, (T)0};
+      if (have) lo[e] = a.st.sol_lo[ubase + k];
+    }
+    if constexpr (ETD) {
+      E[e] = a.st.E[ubase + k];
+      E2[e] = a.st.E2[ubase + k];
+      ze[e] = a.st.zeta[ubase + k];
+      al[e] = a.st.alpha[ubase + k];
+      be[e] = a.st.beta[ubase + k];
+      ga[e] = a.st.gam[ubase + k];
+    } else {
+      L[e] = (T)linear_op(a.st.g, opm, a.st.nkappah, k, 0, 0);
+    }
+    fil[e] = a.st.filtered ? filter_value(a.st.g, a.st.f_order, a.st.f_innerK, a.st.f_decay, k, 0, 0) : 1.0;
+  }
+
+  // N = R2C(-u C2R(i kr x)) of the stage input x
+  auto calcN = [&](const cpx<T>(&x)[R + 1], cpx<T>(&N)[R + 1]) {
+    cpx<T> z[R];
+    lds_sync(kWave);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int k = j + q * P;
+      z[q] = times_ik(x[q], (T)(k * a.kscale_x));
+      lds[lay.idx(0, k)] = z[q];
+    }
+    if (nyq) lds[lay.idx(0, M)] = times_ik(x[R], (T)(M * a.kscale_x));
+    lds_sync(kWave);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int k = j + q * P;
+      z[q] = c2r_pre(z[q], lds[lay.idx(0, M - k)], twl[k], sc, k == 0);
+    }
+    line_fft<T, M, R, +1, LayLine>(z, lds, lay, 0, j, twl, 2, kWave);
+#pragma unroll
+    for (int q = 0; q < R; ++q) z[q] = {-u[q].re * z[q].re, -u[q].im * z[q].im};
+    line_fft<T, M, R, -1, LayLine>(z, lds, lay, 0, j, twl, 2, kWave);
+    lds_sync(kWave);
+#pragma unroll
+    for (int q = 0; q < R; ++q) lds[lay.idx(0, j + q * P)] = z[q];
+    lds_sync(kWave);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int k = j + q * P;
+      // lane 0's partner of k = 0 is not used
+      const cpx<T> Zm = lds[lay.idx(0, k == 0 ? 0 : M - k)];
+      N[q] = k == 0 ? cpx<T>{z[q].re + z[q].im, (T)0} : r2c_post(z[q], Zm, twl[k]);
+    }
+    N[R] = nyq ? cpx<T>{z[0].re - z[0].im, (T)0} : cpx<T>{(T)0, (T)0};
+  };
+
+#pragma unroll 1
+  for (int step = 0; step < a.nsteps; ++step) {
+    cpx<T> x[R + 1], N[R + 1];
+#pragma unroll
+    for (int e = 0; e <= R; ++e) x[e] = s[e];
+    if constexpr (!ETD) {
+      // as rk4_load / rk4_finish, the operands in registers: sp is the FP64 form's sol after
+      // the third stage
+      cpx<T> ac[R + 1], sp[kMixed ? 1 : R + 1];
+#pragma unroll 1
+      for (int stage = 0; stage < 4; ++stage) {
+        calcN(x, N);
+        switch (stage) {
+          case 0:
+#pragma unroll
+            for (int e = 0; e <= R; ++e) {
+              const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
+              ac[e] = rhs;
+              x[e] = {s[e].re + h2 * rhs.re, s[e].im + h2 * rhs.im};
+            }
+            break;
+          case 1:
+#pragma unroll
+            for (int e = 0; e <= R; ++e) {
+              const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
+              ac[e] = {ac[e].re / (T)6 + rhs.re / (T)3, ac[e].im / (T)6 + rhs.im / (T)3};
+              x[e] = {s[e].re + h2 * rhs.re, s[e].im + h2 * rhs.im};
+            }
+            break;
+          case 2:
+#pragma unroll
+            for (int e = 0; e <= R; ++e) {
+              const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
+              ac[e] = {ac[e].re + rhs.re / (T)3, ac[e].im + rhs.im / (T)3};
+              x[e] = {s[e].re + dt * rhs.re, s[e].im + dt * rhs.im};
+              if constexpr (!kMixed) sp[e] = {s[e].re + dt * ac[e].re, s[e].im + dt * ac[e].im};
+            }
+            break;
+          default:
+#pragma unroll
+            for (int e = 0; e <= R; ++e) {
+              const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
+              if constexpr (!kMixed) {
+                s[e] = {sp[e].re + dt * (rhs.re / (T)6), sp[e].im + dt * (rhs.im / (T)6)};
+                if (a.st.filtered) s[e] = {(T)fil[e] * s[e].re, (T)fil[e] * s[e].im};
+              } else {
+                const cpx<T> tot = {ac[e].re + rhs.re / (T)6, ac[e].im + rhs.im / (T)6};
+                T hr, lr, hi, li;
+                comp_add(s[e].re, lo[e].re, dt * tot.re, hr, lr);
+                comp_add(s[e].im, lo[e].im, dt * tot.im, hi, li);
+                if (a.st.filtered) {
+                  const double xr = ((double)hr + (double)lr) * fil[e], xi = ((double)hi + (double)li) * fil[e];
+                  hr = (T)xr;
+                  hi = (T)xi;
+                  lr = (T)(xr - (double)hr);
+                  li = (T)(xi - (double)hi);
+                }
+                s[e] = {hr, hi};
+                lo[e] = {lr, li};
+              }
+            }
+        }
+      }
+    } else {
+      // as etd_load / etd_finish; pr, pi: the partial update between the last two stages
+      cpx<T> n1[R + 1], n2[R + 1], s1[R + 1];
+      double pr[R + 1], pi[R + 1];
+      auto state = [&](int e, double& re, double& im) {
+        re = (double)s[e].re;
+        im = (double)s[e].im;
+        if constexpr (kMixed) {
+          re += (double)lo[e].re;
+          im += (double)lo[e].im;
+        }
+      };
+#pragma unroll 1
+      for (int stage = 0; stage < 4; ++stage) {
+        calcN(x, N);
+#pragma unroll
+        for (int e = 0; e <= R; ++e) {
+          const double nre = (double)N[e].re, nim = (double)N[e].im;
+          if (stage <= 1) {
+            double sr, si;
+            state(e, sr, si);
+            x[e] = {(T)(E2[e] * sr + ze[e] * nre), (T)(E2[e] * si + ze[e] * nim)};
+            if (stage == 0) {
+              n1[e] = N[e];
+              s1[e] = x[e];
+            } else {
+              n2[e] = N[e];
+            }
+          } else if (stage == 2) {
+            double sr, si;
+            state(e, sr, si);
+            x[e] = {(T)(E2[e] * (double)s1[e].re + ze[e] * (2.0 * nre - (double)n1[e].re)),
+                    (T)(E2[e] * (double)s1[e].im + ze[e] * (2.0 * nim - (double)n1[e].im))};
+            const double b2 = 2.0 * be[e];
+            pr[e] = E[e] * sr + al[e] * (double)n1[e].re + b2 * ((double)n2[e].re + nre);
+            pi[e] = E[e] * si + al[e] * (double)n1[e].im + b2 * ((double)n2[e].im + nim);
+          } else {
+            const double sr = (pr[e] + ga[e] * nre) * fil[e], si = (pi[e] + ga[e] * nim) * fil[e];
+            s[e] = {(T)sr, (T)si};
+            if constexpr (kMixed) lo[e] = {(T)(sr - (double)s[e].re), (T)(si - (double)s[e].im)};
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e <= R; ++e) {
+    if (e < R || nyq) {
+      a.st.sol[ubase + kof(e)] = s[e];
+      if constexpr (kMixed) a.st.sol_lo[ubase + kof(e)] = lo[e];
+    }
+  }
+}
+
+// The compiled kernel for nx points (null when there is none); threads = its workgroup size.
+const void* line_kernel(bool dbl, bool etd, int nx, int* threads);
+
+}  // namespace ptf
