@@ -193,6 +193,9 @@ struct Slot {
     const int P = N / r;
     return P <= 64 && 64 % P == 0 && (dbl || P <= 32);
   }
+  bool wg_only(int r) const {
+    return !dbl && is_col() && brick > 0 && fixed_threads == 0 && r > 0 && !((kind == 6 || kind == 8) && par) && N == 64 * r;
+  }
   int wave_lines() const { return wave_ok(R) && !wg ? 1 : 0; }
   bool has_occ() const { return kind == 3 || kind == 6 || kind == 8 || kind == 13 || kind == 14; }
   // par: the input-parallel advection form (kinds 13, 14) or the pipelined persistent
@@ -224,7 +227,10 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
   if (wg) {
     Slot t = s;
     t.par = par;
-    if (!t.wave_ok(R)) return false;   // the workgroup form only where the wavefront one applies
+    // the workgroup form only where the wavefront one applies, or (FP32 lines of 64 threads)
+    // where it is the only one
+    if (!t.wave_ok(R) && !t.wg_only(R)) return false;
+    if (!t.wave_ok(R)) wg = 0;
   }
   if (s.brick > 0) {
     // a bricked line needs whole bricks per thread group; bricked rows go in whole bricks
@@ -244,8 +250,108 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
   return true;
 }
 
-// default variant: first valid (R, W) in preference order
+// ---- default variant -------------------------------------------------------------------
+// The variant a slot starts with (a problem runs with it unless ptf_autotune or a
+// set_variant call picks another).  For power-of-two lines it follows from the line length
+// and the size of the launch; the lines of the rule lie where the timings of every compiled
+// variant cross (33 problems: 1D 32..2048, 2D 64^2..2048^2 and oblong, 3D 32^3..256^3, batches
+// of members; the rule's choice is within 2 % of the fastest on average, 20 % at worst):
+//  * radix 4 while a launch has fewer wavefronts than the chip holds or a line is short: it
+//    gives the most threads per line (2D 256^2 FP64: x_advect 4.9 us against 35 us at radix
+//    16).  Long lines (rows from 1024, columns from 2048 points) and fields that stream from
+//    HBM take radix 8: fewer passes (3D 256^3 FP64 z kernel 134 us, radix 4 154 us).
+//  * the fewest lines per block that still fill a wavefront, so that a small field spreads
+//    over all CUs (256 of them); wider where there are blocks to spare, to read whole bricks
+//    (rows: 4 of 8; 8 where a 3D field streams from HBM: 141 against 162 us at 256^3).
+//  * the 3-waves/SIMD build of the stage kernels where a launch is more than latency (FP32
+//    128^3 ETDRK4: 18 against 25 us), the default budget below (2D 256^2 FP32: 5.9 against 6.1).
+//  * advection with the input rows side by side (par) where LDS holds every block a CU
+//    gets, except where rows of 256 and more points come in threes or an FP32 launch already
+//    fills the chip (one after another: 3D 256^3 FP64 141 against 189 us).
+struct Variant {
+  int R, W, occ, par, wg;
+};
+static constexpr long long kCus = 256;
+
+static bool pow2_len(int n) { return n > 0 && (n & (n - 1)) == 0; }
+static int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+
+static Variant row_default(const Slot& s) {
+  const int M = s.N / 2;
+  const long long rows = s.lines * s.members;
+  const long long elems = rows * M, bytes = elems * (s.dbl ? 16 : 8);
+  if (s.kind == K_ROW_C2R || s.kind == K_ROW_R2C) {
+    // contiguous rows need no wide blocks (256^3 FP32 inverse: 76 us at 4 rows, 89 at 8)
+    if (s.brick == 0) return s.N > 1024 ? Variant{8, 2, 0, 0, 0} : Variant{4, 4, 0, 0, 0};
+    if (s.N >= 1024) return {8, s.N >= 2048 ? 8 : 4, 0, 0, 0};
+    return {4, s.N <= 256 ? 8 : 4, 0, 0, 0};
+  }
+  if (s.kind == K_ROW_ADV1) return {4, clampi(256 / M, 1, 16), 0, 0, 0};
+  const int nin = s.kind == K_ROW_ADV3 ? 3 : 2;
+  const bool stream3 = nin == 3 && bytes >= (1LL << 26);
+  const int R = s.N >= 1024 && elems >= (1LL << 18) ? 8 : 4;
+  // LDS of the blocks that share a CU (at least one, at most two asked for)
+  const long long cb = s.dbl ? 16 : 8;
+  const long long tw = s.N > 2048 ? 0 : (s.N * cb > 16384 ? s.N * cb / 2 : s.N * cb);
+  auto fits = [&](int W, int par) {
+    const long long lds = (par ? nin : 1) * W * (M + 1) * cb + tw;
+    const long long blocks = (rows + W - 1) / W;
+    return lds * (blocks > kCus ? 2 : 1) <= 163840;
+  };
+  int W = clampi(64 * R / M, 1, 16);
+  int par = (W * (M / R)) % 64 == 0 && !(nin == 3 && s.N > 128) && !(!s.dbl && elems >= (1LL << 21)) && fits(W, 1);
+  auto widen = [&]() {
+    while (W < (stream3 ? 8 : 4) && rows / (2 * W) >= kCus && fits(2 * W, par)) W *= 2;
+  };
+  widen();
+  if (par && s.N >= 2048 && W < 2) {
+    par = 0;   // a block of one such row leaves its lines' neighbours to others
+    widen();
+  }
+  return {R, W, !par && (s.dbl ? nin == 3 : elems >= (1LL << 21)) ? 3 : 0, par, 0};
+}
+
+static Variant col_default(const Slot& s) {
+  const int N = s.N;
+  const long long elems = s.lines * s.other * s.members * N, bytes = elems * (s.dbl ? 16 : 8);
+  const bool stream = bytes >= (1LL << 26);
+  switch (s.kind) {
+    case K_COL_D2:
+      if (s.dbl) return stream ? Variant{8, 8, 3, 0, 0} : Variant{4, N <= 32 ? 8 : 4, 0, 0, 0};
+      return N < 64 || (N >= 256 && stream) ? Variant{4, 8, 0, 0, 0} : Variant{8, 8, 0, 0, 0};
+    case K_COL_FWD:
+    case K_COL_INV:
+      return s.dbl || N <= 32 ? Variant{4, 8, 0, 0, 0} : Variant{8, 8, 0, 0, 0};
+    case K_COL_FLOWSYN:
+      return N >= 2048 ? Variant{8, 1, 0, 0, 0} : Variant{4, clampi(512 / N, 1, 8), 0, 0, 0};
+    default: break;
+  }
+  // stage kernels (and the prologue's inverse pair): the 3-waves/SIMD build where the launch
+  // is more than latency
+  const bool big = elems >= (1LL << 19);
+  const int occ = s.has_occ() && (big || N >= 2048) ? 3 : 0;
+  if (N >= 2048) return {8, 1, occ, 0, 0};
+  if (N > 256) return N <= 512 && bytes >= (1LL << 25) ? Variant{8, s.dbl ? 2 : 1, occ, 0, 0} : Variant{4, 1, occ, 0, 0};
+  if (N > 128) {
+    if (s.dbl ? bytes >= (1LL << 27) : bytes >= (1LL << 26)) return {8, 8, occ, 0, 1};
+    return {4, bytes >= (1LL << 24) ? 4 : 2, occ, 0, 0};
+  }
+  if (N > 64) return {4, big ? 4 : 2, occ, 0, big && !s.dbl ? 1 : 0};
+  if (N < 64) return {4, 8, occ, 0, 0};
+  return !s.dbl && bytes >= (1LL << 24) ? Variant{8, 8, occ, 0, 0} : Variant{4, 4, occ, 0, 0};
+}
+
+// the default variant, else the first valid (R, W) in preference order
 static int pick_default(Slot& s) {
+  if (pow2_len(s.N) && s.N >= 16) {
+    Variant v = s.is_col() ? col_default(s) : row_default(s);
+    if (v.wg && !s.wave_ok(v.R)) v.wg = 0;
+    // a width with no compiled kernel at this length: the next narrower, then wider one
+    for (int W = v.W; W >= 1; W /= 2)
+      if (choose_variant(s, v.R, W, v.occ, W == v.W ? v.par : 0, v.wg)) return PTF_OK;
+    for (int W = v.W * 2; W <= 64; W *= 2)
+      if (choose_variant(s, v.R, W, v.occ, 0, v.wg)) return PTF_OK;
+  }
   const int* widths = s.is_col() ? kColWidths : kRowWidths;
   const int nw = s.is_col() ? kNumColWidths : kNumRowWidths;
   for (int R : kRadices) {
@@ -1374,7 +1480,7 @@ static int autotune_group(Group& g, hipStream_t st) {
               bool ok = true;
               for (Slot* o : same) {
                 Slot trial = *o;
-                if (!choose_variant(trial, R, widths[wi], occ, par, wg)) {
+                if (!choose_variant(trial, R, widths[wi], occ, par, wg) || trial.wg != wg) {
                   ok = false;
                   break;
                 }
