@@ -476,6 +476,9 @@ static int dalloc(DevBuf& b, size_t nbytes) {
 }
 
 
+// blocks of the diagnostics' partial sums: Group::red holds a pair for each, and a record
+static constexpr int kDiagBlocks = 1024;
+
 // ---------------------------------------------------------------------------
 // group of B problems on one grid
 // ---------------------------------------------------------------------------
@@ -1118,7 +1121,7 @@ static int group_init_once(Group& g, const ptf_desc* descs, int count, int lb, b
   for (int i = 0; i < g.ndim; ++i) HIPCHK(hipMemset(g.flow[i].p, 0, Rb));
   CHK(dalloc(g.phys, (size_t)g.nR * g.esz));
   CHK(dalloc(g.spec, (size_t)g.nS * cs));
-  CHK(dalloc(g.red, 2 * sizeof(double) * 1024));
+  CHK(dalloc(g.red, (2 * kDiagBlocks + 2) * sizeof(double)));
   if (g.flow_kind == PTF_FLOW_SPECTRAL) {
     CHK(dalloc(g.fs[0], (size_t)g.nS * cs));
     CHK(dalloc(g.fs[1], (size_t)g.nS * cs));
@@ -2227,53 +2230,53 @@ int ptf_get_L(ptf_problem* prob, double* L) {
   return PTF_OK;
 }
 
-static int diagnostics_group(Group& g, int member, hipStream_t st, double* mass, double* var) {
-  const size_t cs = 2 * g.esz;
-  const char* base = (const char*)g.sol.p + (size_t)member * g.nS * cs;
+// Launches that write (mass, variance) of a member into rec[0..1] on the device.  Enough
+// blocks for four elements a thread, at most kDiagBlocks.
+static int launch_diag(Group& g, int member, hipStream_t st, double* rec) {
+  const size_t off = (size_t)member * g.nS * 2 * g.esz;
+  const char* base = (const char*)g.sol.p + off;
   // the mixed form's state is the compensated pair sol + sol_lo: both enter the FP64 sums
-  const char* lo = g.sol_lo.p ? (const char*)g.sol_lo.p + (size_t)member * g.nS * cs : nullptr;
-  double s0re = 0, s0im = 0;
+  const char* lo = g.sol_lo.p ? (const char*)g.sol_lo.p + off : nullptr;
+  const int blocks = (int)std::min<long long>(kDiagBlocks, (g.nS + 1023) / 1024);
+  double* part = (double*)g.red.p;
   if (g.dbl) {
-    double v[2];
-    HIPCHK(hipMemcpyAsync(v, base, 16, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    s0re = v[0];
-    s0im = v[1];
+    hipLaunchKernelGGL(variance_partial_kernel<double>, dim3(blocks), dim3(256), 0, st, (const cpx<double>*)base,
+                       (const cpx<double>*)nullptr, g.nS, g.nxh, g.lb, part);
+    hipLaunchKernelGGL(diag_record_kernel<double>, dim3(1), dim3(256), 0, st, (const cpx<double>*)base,
+                       (const cpx<double>*)nullptr, (const double*)part, blocks, (double)g.nR, rec);
   } else {
-    float v[2], w[2] = {0.f, 0.f};
-    HIPCHK(hipMemcpyAsync(v, base, 8, hipMemcpyDeviceToHost, st));
-    if (lo) HIPCHK(hipMemcpyAsync(w, lo, 8, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    s0re = (double)v[0] + (double)w[0];
-    s0im = (double)v[1] + (double)w[1];
+    hipLaunchKernelGGL(variance_partial_kernel<float>, dim3(blocks), dim3(256), 0, st, (const cpx<float>*)base,
+                       (const cpx<float>*)lo, g.nS, g.nxh, g.lb, part);
+    hipLaunchKernelGGL(diag_record_kernel<float>, dim3(1), dim3(256), 0, st, (const cpx<float>*)base,
+                       (const cpx<float>*)lo, (const double*)part, blocks, (double)g.nR, rec);
   }
-  if (mass) *mass = s0re;
-  if (var) {
-    const int blocks = 1024;
-    if (g.dbl)
-      hipLaunchKernelGGL(variance_partial_kernel<double>, dim3(blocks), dim3(256), 0, st,
-                         (const cpx<double>*)base, (const cpx<double>*)nullptr, g.nS, g.nxh, g.lb,
-                         (double*)g.red.p);
-    else
-      hipLaunchKernelGGL(variance_partial_kernel<float>, dim3(blocks), dim3(256), 0, st,
-                         (const cpx<float>*)base, (const cpx<float>*)lo, g.nS, g.nxh, g.lb,
-                         (double*)g.red.p);
-    HIPCHK(hipGetLastError());
-    std::vector<double> part(2 * blocks);
-    HIPCHK(hipMemcpyAsync(part.data(), g.red.p, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    double sum = 0, comp = 0;
-    for (int i = 0; i < 2 * blocks; ++i) {
-      const double x = part[i];
-      const double t = sum + x;
-      comp += (std::fabs(sum) >= std::fabs(x)) ? (sum - t) + x : (x - t) + sum;
-      sum = t;
+  HIPCHK(hipGetLastError());
+  return PTF_OK;
+}
+
+static int diagnostics_group(Group& g, int member, hipStream_t st, double* mass, double* var) {
+  if (!var) {   // the mass alone is one element of the state
+    if (!mass) return PTF_OK;
+    const size_t cs = 2 * g.esz, off = (size_t)member * g.nS * cs;
+    double v[2] = {0.0, 0.0};
+    float f[2] = {0.f, 0.f};
+    if (g.dbl) {
+      HIPCHK(hipMemcpyAsync(v, (const char*)g.sol.p + off, sizeof(double), hipMemcpyDeviceToHost, st));
+    } else {
+      HIPCHK(hipMemcpyAsync(&f[0], (const char*)g.sol.p + off, sizeof(float), hipMemcpyDeviceToHost, st));
+      if (g.sol_lo.p) HIPCHK(hipMemcpyAsync(&f[1], (const char*)g.sol_lo.p + off, sizeof(float), hipMemcpyDeviceToHost, st));
     }
-    const double dc = s0re * s0re + s0im * s0im;
-    const double tot = (sum - dc) + comp;
-    const double N = (double)g.nR;
-    *var = tot / (N * N);
+    HIPCHK(hipStreamSynchronize(st));
+    *mass = g.dbl ? v[0] : (double)f[0] + (double)f[1];
+    return PTF_OK;
   }
+  double* rec = (double*)g.red.p + 2 * kDiagBlocks;
+  CHK(launch_diag(g, member, st, rec));
+  double h[2];
+  HIPCHK(hipMemcpyAsync(h, rec, sizeof(h), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  if (mass) *mass = h[0];
+  if (var) *var = h[1];
   return PTF_OK;
 }
 
@@ -2304,7 +2307,6 @@ int ptf_step_record(ptf_problem* prob, int64_t nsteps, int64_t every, int64_t ca
   if (want_diag && nrec > 0) rc = dalloc(rec, (size_t)nrec * 2 * sizeof(double));
   if (rc == PTF_OK && c_out && nrec > 0) rc = dalloc(snaps, (size_t)nrec * rsz);
   if (rc != PTF_OK) return rc;
-  const int blocks = 1024;
   int64_t r = 0;
   for (int64_t i = 0; i < nsteps && rc == PTF_OK; ++i) {
     rc = group_step_launches(g, st, prob->t);
@@ -2315,23 +2317,7 @@ int ptf_step_record(ptf_problem* prob, int64_t nsteps, int64_t every, int64_t ca
     if (t_out) t_out[r] = prob->t;
     if (step_out) step_out[r] = prob->step;
     if (want_diag) {
-      double* dst = (double*)rec.p + 2 * r;
-      if (g.dbl) {
-        hipLaunchKernelGGL(variance_partial_kernel<double>, dim3(blocks), dim3(256), 0, st,
-                           (const cpx<double>*)g.sol.p, (const cpx<double>*)nullptr, g.nS, g.nxh,
-                           g.lb, (double*)g.red.p);
-        hipLaunchKernelGGL(diag_record_kernel<double>, dim3(1), dim3(64), 0, st,
-                           (const cpx<double>*)g.sol.p, (const cpx<double>*)nullptr,
-                           (const double*)g.red.p, 2 * blocks, (double)g.nR, dst);
-      } else {
-        hipLaunchKernelGGL(variance_partial_kernel<float>, dim3(blocks), dim3(256), 0, st,
-                           (const cpx<float>*)g.sol.p, (const cpx<float>*)g.sol_lo.p, g.nS, g.nxh,
-                           g.lb, (double*)g.red.p);
-        hipLaunchKernelGGL(diag_record_kernel<float>, dim3(1), dim3(64), 0, st,
-                           (const cpx<float>*)g.sol.p, (const cpx<float>*)g.sol_lo.p,
-                           (const double*)g.red.p, 2 * blocks, (double)g.nR, dst);
-      }
-      if (hipGetLastError() != hipSuccess) rc = fail(PTF_ERR_DEVICE, "diagnostics launch failed");
+      rc = launch_diag(g, 0, st, (double*)rec.p + 2 * r);
     }
     if (rc == PTF_OK && c_out) rc = g_irfft(g, g.sol.p, (char*)snaps.p + (size_t)r * rsz, st);
     ++r;
@@ -2651,7 +2637,6 @@ int ptf_ensemble_diagnostics(ptf_ensemble* ens, int32_t member, double* mass, do
   Group* g;
   int i;
   CHK(member_of(ens, member, &g, &i));
-  if (!g->red.p) CHK(dalloc(g->red, 2 * 1024 * sizeof(double)));
   return diagnostics_group(*g, i, ens->stream, mass, variance);
 }
 
