@@ -4,7 +4,8 @@
 
 The kernel registry (csrc/ptf_registry.hip) is compiled once per
 (precision, kernel kind) so the units build in parallel; csrc/ptf_member.hip holds
-the whole-member step kernels; csrc/ptf_api.hip is the host runtime.  All HIP code is built with packed-FP32 instructions off.
+the whole-member step kernels, csrc/ptf_line.hip the whole-run kernels of 1D problems;
+csrc/ptf_api.hip is the host runtime.  All HIP code is built with packed-FP32 instructions off.
 """
 from __future__ import annotations
 
@@ -53,11 +54,18 @@ def _units():
     obj = os.path.join(OBJDIR, "ptf_member.o")
     units.append((obj, [HIPCC, *COMMON, "-c", os.path.join(CSRC, "ptf_member.hip"), "-o", obj],
                   ["ptf_member.hip", "ptf_member.hpp", *HEADERS]))
+    # the whole-run kernels of 1D problems, per precision and stepper family
+    for t, tn in PRECS:
+        for etd in (0, 1):
+            obj = os.path.join(OBJDIR, f"ptf_line_{tn}_{etd}.o")
+            units.append((obj, [HIPCC, *COMMON, f"-DPTF_T={t}", f"-DPTF_TNAME={tn}", f"-DPTF_ETD={etd}",
+                                "-c", os.path.join(CSRC, "ptf_line.hip"), "-o", obj],
+                          ["ptf_line.hip", "ptf_line.hpp", *HEADERS]))
     # the heaviest units first, so that they do not end up on the critical path last
     units.sort(key=lambda u: -_weight(u[0]))
     obj = os.path.join(OBJDIR, "ptf_api.o")
     units.append((obj, [HIPCC, *COMMON, "-c", os.path.join(CSRC, "ptf_api.hip"), "-o", obj],
-                  ["ptf_api.hip", *API_HEADERS, "ptf_member.hpp", os.path.join(INCLUDE, "ptf.h")]))
+                  ["ptf_api.hip", *API_HEADERS, "ptf_line.hpp", "ptf_member.hpp", os.path.join(INCLUDE, "ptf.h")]))
     return units
 
 
@@ -119,7 +127,7 @@ def build_asan(verbose: bool = True) -> str:
     Load it with the clang ASan runtime preloaded (see tests/test_sanitizer.py); it is for
     the CPU tests of the boundary (argument checks, error paths, host buffers)."""
     units = _units()
-    regs = [o for o, _, _ in units if os.path.basename(o).startswith(("reg_", "ptf_member"))]
+    regs = [o for o, _, _ in units if os.path.basename(o).startswith(("reg_", "ptf_member", "ptf_line"))]
     missing = [o for o in regs if not os.path.exists(o)]
     if missing:
         raise RuntimeError("build the library first (missing " + os.path.basename(missing[0]) + ")")
