@@ -354,8 +354,38 @@ static Variant col_default(const Slot& s) {
   return !s.dbl && bytes >= (1LL << 24) ? Variant{8, 8, occ, 0, 0} : Variant{4, 4, occ, 0, 0};
 }
 
+// Lengths that are no powers of two (2^a m): the narrow register layout, whose few elements
+// per lane do not spill, at the width that fills a wavefront, twice that where a field streams
+// (FP32 from 4 MB, FP64 from 64 MB: 200^3 stage kernels 56 against 85 us and 89 against 105).
+// Columns whose wide layout saves three passes or more (2^a 3 from 96 points on; FP32 also
+// 2^a 5, which spills in FP64) take it for fields from 16 MB: 192^3 FP64 54 against 65 us.
+static Variant mixed_default(const Slot& s) {
+  const int L = s.is_col() ? s.N : s.N / 2;
+  const int en = line_e_narrow(L), ew = line_e(L);
+  const long long elems = s.lines * s.other * s.members * L, bytes = elems * (s.dbl ? 16 : 8);
+  if (s.is_col()) {
+    if (radix_plan(L, en).n - radix_plan(L, ew).n >= 3 && bytes >= (1LL << 24) && (!s.dbl || L % 5 != 0))
+      return {ew, reduced_width(L / ew, 64), 0, 0, 0};
+    int W = narrow_width(L / en, 2);
+    if (2 * W * (L / en) <= 256 && bytes >= (s.dbl ? (s.kind == K_COL_D2 ? 1LL << 40 : 1LL << 26) : 1LL << 22)) W *= 2;
+    return {en, W, 0, 0, 0};
+  }
+  const int W = narrow_width(L / en, 1);
+  const bool adv = s.kind == K_ROW_ADV2 || s.kind == K_ROW_ADV3;
+  const int par = adv && (W * (L / en)) % 64 == 0 && !(s.kind == K_ROW_ADV3 && s.N > 128) &&
+                  !(!s.dbl && elems >= (1LL << 21));
+  return {en, W, 0, par, 0};
+}
+
 // the default variant, else the first valid (R, W) in preference order
 static int pick_default(Slot& s) {
+  const int len = s.is_col() ? s.N : s.N / 2;
+  if (!pow2_len(len) && line_e(len) > 0) {
+    const Variant v = mixed_default(s);
+    if (v.par && choose_variant(s, v.R, v.W, 0, 1)) return PTF_OK;
+    if (choose_variant(s, v.R, v.W)) return PTF_OK;
+    if (choose_variant(s, line_e_narrow(len), narrow_width(len / line_e_narrow(len), s.is_col() ? 2 : 1))) return PTF_OK;
+  }
   if (pow2_len(s.N) && s.N >= 16) {
     Variant v = s.is_col() ? col_default(s) : row_default(s);
     if (v.wg && !s.wave_ok(v.R)) v.wg = 0;
@@ -908,8 +938,8 @@ static bool build_member_slot(Group& g) {
 // 1D problems advance by whole runs of steps in one launch, a workgroup per member
 // (line_run_kernel), where a kernel is compiled for the length.  The four stage launches of a
 // step are kept for callers that time or select them one by one.  Always the faster of the
-// two: a step in a run takes 6.5 us against 23.6 by its four launches at 128 points FP64, 30
-// against 127 at 1000, 36 against 56 at 4096 (the nearest); FP32 ETDRK4 12 against 34 at 1024.
+// two: a step in a run takes 6.5 us against 23.6 by its four launches at 128 points FP64, 25
+// against 114 at 1000, 36 against 56 at 4096 (the nearest); FP32 ETDRK4 12 against 34 at 1024.
 // One step a call: 21 against 38 us at 128, 52 against 68 at 4096.
 template <typename T>
 static void build_line_slot(Group& g) {
@@ -1092,7 +1122,11 @@ static int group_init(Group& g, const ptf_desc* descs, int count, bool allow_bri
   int lb = 0;
   if (allow_brick && d.ndim >= 2) {
     const long long nlast = d.ndim == 3 ? d.n[2] : d.n[1];
-    if (nlast >= 64 && nlast % 8 == 0) lb = 3;   // whole bricks of 8 planes
+    // whole bricks of 8 planes (of a length that is no power of two only where the wide register
+    // layout can hold bricked lines)
+    const bool pow2 = pow2_len((int)nlast);
+    const int e = pow2 ? 1 : line_e((int)nlast);
+    if (nlast >= 64 && nlast % 8 == 0 && (pow2 || (e > 0 && (nlast / e) % 8 == 0))) lb = 3;
   }
   int rc = group_init_once(g, descs, count, lb, plan_only);
   if (rc == PTF_ERR_UNSUPPORTED && lb > 0) rc = group_init_once(g, descs, count, 0, plan_only);

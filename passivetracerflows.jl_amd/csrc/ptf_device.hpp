@@ -20,7 +20,7 @@
 // natural-layout registers.  So the first pass (Ns = 1, no twiddles) works on
 // registers, and the last pass (Ns*Rp = N) writes its outputs back to the
 // registers it read.  Powers of two use N = R0 * R^K (R0 <= R first); other
-// lengths 2^a 3^b 5^c use radices 2, 3, 4, 5, 8, 16 that divide E.
+// lengths 2^a 3^b 5^c use the largest of the radices 2..6, 8, 10, 12, 16, 20 that divide E.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -186,6 +186,39 @@ __device__ __forceinline__ void dft5(cpx<T>* a) {
 }
 
 template <int R, int DIR, typename T>
+__device__ __forceinline__ void dft(cpx<T>* a);
+
+// DFT of length N1 N2, N1 and N2 coprime, as N2 DFTs of length N1 and N1 of length N2 with no
+// twiddles between them (Good 1958): input n = (N2 n1 + N1 n2) mod N, output the k with
+// k = k1 mod N1 and k = k2 mod N2.
+constexpr int inv_mod(int a, int m) {
+  for (int x = 1; x < m; ++x)
+    if (a * x % m == 1) return x;
+  return 0;
+}
+template <int N1, int N2, int DIR, typename T>
+__device__ __forceinline__ void dft_coprime(cpx<T>* a) {
+  constexpr int N = N1 * N2;
+  constexpr int u1 = N2 * inv_mod(N2 % N1, N1), u2 = N1 * inv_mod(N1 % N2, N2);
+  cpx<T> b[N2][N1];
+#pragma unroll
+  for (int n2 = 0; n2 < N2; ++n2) {
+#pragma unroll
+    for (int n1 = 0; n1 < N1; ++n1) b[n2][n1] = a[(N2 * n1 + N1 * n2) % N];
+    dft<N1, DIR>(b[n2]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < N1; ++k1) {
+    cpx<T> c[N2];
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) c[n2] = b[n2][k1];
+    dft<N2, DIR>(c);
+#pragma unroll
+    for (int k2 = 0; k2 < N2; ++k2) a[(u1 * k1 + u2 * k2) % N] = c[k2];
+  }
+}
+
+template <int R, int DIR, typename T>
 __device__ __forceinline__ void dft(cpx<T>* a) {
   if constexpr (R == 2) dft2<DIR>(a[0], a[1]);
   else if constexpr (R == 4) dft4<DIR>(a[0], a[1], a[2], a[3]);
@@ -193,6 +226,10 @@ __device__ __forceinline__ void dft(cpx<T>* a) {
   else if constexpr (R == 16) dft16<DIR>(a);
   else if constexpr (R == 3) dft3<DIR>(a);
   else if constexpr (R == 5) dft5<DIR>(a);
+  else if constexpr (R == 6) dft_coprime<2, 3, DIR>(a);
+  else if constexpr (R == 10) dft_coprime<2, 5, DIR>(a);
+  else if constexpr (R == 12) dft_coprime<4, 3, DIR>(a);
+  else if constexpr (R == 20) dft_coprime<4, 5, DIR>(a);
   else static_assert(R == 2, "unsupported radix");
 }
 
@@ -207,12 +244,12 @@ struct RadixPlan {
 constexpr RadixPlan radix_plan(int N, int E) {
   RadixPlan p{0, {}};
   if (N < 2 || E < 2 || N % E != 0) return p;
-  const int pref[6] = {16, 8, 5, 4, 3, 2};
+  const int pref[10] = {20, 16, 12, 10, 8, 6, 5, 4, 3, 2};
   int tmp[24] = {};
   int k = 0, rest = N;
   while (rest > 1) {
     int pick = 0;
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < 10; ++i) {
       if (E % pref[i] == 0 && rest % pref[i] == 0) {
         pick = pref[i];
         break;
@@ -239,7 +276,7 @@ constexpr int fft_barriers(int N, int E) {
   return n >= 2 ? 2 * n - 2 : 0;
 }
 
-// Elements per thread of the one register layout compiled for a line length N that is
+// Elements per thread of the wide register layout compiled for a line length N that is
 // not a power of two: N = 2^a 3^b 5^c with E = 2^min(a,2) times the product of the
 // distinct odd primes (2^min(a,1) times it when both 3 and 5 divide N), at most 30;
 // 0 when N has another prime factor or is a power of two.
@@ -261,6 +298,18 @@ constexpr int line_e(int N) {
   if (n != 1 || odd == 1) return 0;
   const int e = (odd < 15 ? (1 << (a < 2 ? a : 2)) : (1 << (a < 1 ? a : 1))) * odd;
   return e <= 30 && fft_ok(N, e) ? e : 0;
+}
+
+// Elements per thread of the narrow layout: just the odd prime, doubled where N is even (6 or
+// 10; 3 or 5 for odd N).  It leaves the registers free that the wide one spills: 400 x 216
+// FP64, x pass 62 -> 10 us, fused y kernel 20 -> 8 us.  (The wide layout has fewer passes, 3
+// instead of 6 at 192 points, and stays the better one where long fields stream from HBM.)
+constexpr int line_e_narrow(int N) {
+  const int w = line_e(N);
+  if (w == 0) return 0;
+  const int odd = N % 3 == 0 ? 3 : 5;
+  const int e = N % 2 == 0 ? 2 * odd : odd;
+  return N % 15 != 0 && fft_ok(N, e) ? e : w;
 }
 
 // LDS layouts: line c, element i

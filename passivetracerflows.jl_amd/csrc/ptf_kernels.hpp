@@ -97,6 +97,21 @@ constexpr int min_waves(int threads, int lds, int occ = 0) {
   return w < want ? w : want;
 }
 
+// Lines (or rows) per block of the narrow mixed-radix layout: the smallest power of two, at
+// least wmin and at most 16, that fills a wavefront with P threads a line.
+constexpr int narrow_width(int P, int wmin) {
+  int w = wmin;
+  while (w < 16 && w * P < 64) w *= 2;
+  return w;
+}
+
+// ... and of the wide one: the largest power of two, at most wmax, within 128 threads.
+constexpr int reduced_width(int P, int wmax) {
+  int w = 1;
+  while (w * 2 <= wmax && w * 2 * P <= 128) w *= 2;
+  return w;
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs of the device, each
 // with its own L2.  Renumber the grid so that XCD k runs a contiguous range of
 // logical blocks (x fastest, then y, then z): neighbouring tiles, which share

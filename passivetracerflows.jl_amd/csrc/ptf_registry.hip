@@ -58,17 +58,21 @@ constexpr int row_nin(int k) { return k == K_ROW_ADV2 ? 2 : k == K_ROW_ADV3 ? 3 
 // kinds that are also built with a 3-waves/SIMD register budget (OCC = 3)
 constexpr bool has_occ(int k) { return k == 3 || k == 6 || k == 8 || k == 13 || k == 14; }
 
-// Lengths that are not powers of two are compiled with one register layout (R =
-// line_e(N) elements per thread), the default register budget, and one width: the
-// largest power of two (at most wmax) that keeps a block within 128 threads.
+// Lengths that are not powers of two are compiled at the default register budget with two
+// register layouts: the wide one (R = line_e(N) elements per thread) at one width, the largest
+// power of two (at most wmax) that keeps a block within 128 threads, and, for the kinds that
+// carry a step, the narrow one (line_e_narrow) at two widths: the smallest that fills a
+// wavefront (columns: at least 2, to share cache lines) and twice that.
 constexpr bool is_pow2_len(int n) { return n > 0 && (n & (n - 1)) == 0; }
-constexpr int reduced_width(int P, int wmax) {
-  int w = 1;
-  while (w * 2 <= wmax && w * 2 * P <= 128) w *= 2;
-  return w;
+constexpr bool has_narrow(int k) {
+  return k == K_COL_FWD || k == K_COL_INV || k == K_COL_D2 || k == K_COL_FLOWSYN || k == K_COL_STAGE_D1 ||
+         k == K_COL_STAGE_D1_RK4 || k == K_ROW_C2R || k == K_ROW_R2C || k == K_ROW_ADV2 || k == K_ROW_ADV3;
 }
-constexpr bool reduced_ok(int N, int R, int width, int wmax, int P, int OCC) {
-  return R == line_e(N) && OCC == 0 && width == reduced_width(P, wmax);
+constexpr bool reduced_ok(int N, int R, int width, int wmax, int P, int OCC, int kind) {
+  if (OCC != 0) return false;
+  if (R == line_e(N) && width == reduced_width(P, wmax)) return true;
+  const int w = narrow_width(P, kind < 10 ? 2 : 1);
+  return has_narrow(kind) && R == line_e_narrow(N) && (width == w || width == 2 * w);
 }
 
 template <typename T, int N, int R, int TX, int KIND, int OCC>
@@ -76,7 +80,7 @@ const void* colp() {
   constexpr int P = N / R;
   constexpr bool ok = R <= N && (R >= 4 || !is_pow2_len(N)) && N % R == 0 && fft_ok(N, R) &&
                       TX * P >= 16 && TX * P <= 1024 &&
-                      (is_pow2_len(N) || reduced_ok(N, R, TX, 64, P, OCC)) &&
+                      (is_pow2_len(N) || reduced_ok(N, R, TX, 64, P, OCC, KIND)) &&
                       (long long)col_lds_elems<T, N, R, TX, col_mode(KIND)>() * (long long)sizeof(cpx<T>) <= 163840;
   if constexpr (ok) {
     return reinterpret_cast<const void*>(
@@ -92,7 +96,7 @@ const void* rowp() {
   constexpr int P = M / R;
   constexpr bool ok = R <= M && (R >= 4 || !is_pow2_len(M)) && M % R == 0 && fft_ok(M, R) &&
                       NL * P >= 16 && NL * P <= 1024 &&
-                      (is_pow2_len(M) || reduced_ok(M, R, NL, 16, P, OCC)) &&
+                      (is_pow2_len(M) || reduced_ok(M, R, NL, 16, P, OCC, KIND)) &&
                       (long long)NL * (M + 1) * (long long)sizeof(cpx<T>) + row_tw_bytes<T, NX>() <= 163840;
   if constexpr (ok) {
     return reinterpret_cast<const void*>(&row_kernel<T, NX, R, NL, row_mode(KIND), row_nin(KIND), OCC>);
@@ -108,7 +112,8 @@ const void* rowpar() {
     constexpr int NIN = row_nin(KIND);
     constexpr int M = NX / 2;
     constexpr int P = M / R;
-    constexpr bool ok = is_pow2_len(M) && R <= M && R >= 4 && (NL * P) % 64 == 0 &&
+    constexpr bool ok = ((is_pow2_len(M) && R >= 4) || (R == line_e_narrow(M) && reduced_ok(M, R, NL, 16, P, OCC, KIND))) && R <= M &&
+                        (NL * P) % 64 == 0 &&
                         NIN * NL * P <= 1024 &&
                         adv_par_lds<T, NX, R, NL, NIN>() <= 163840;
     if constexpr (ok) {
@@ -218,6 +223,9 @@ const void* by_r(int R, int W) {
     }
   } else if constexpr (line_e(L) > 0) {
     if (R == line_e(L)) return by_w<T, N, line_e(L), KIND>(W);
+    if constexpr (line_e_narrow(L) != line_e(L) && has_narrow(KIND)) {
+      if (R == line_e_narrow(L)) return by_w<T, N, line_e_narrow(L), KIND>(W);
+    }
     return nullptr;
   } else {
     return nullptr;
@@ -244,7 +252,7 @@ const void* by_n(int N, int R, int W) {
       case 512: return in_part<T, 512, KIND, 6>(R, W);
       case 1024: return in_part<T, 1024, KIND, 7>(R, W);
       case 2048: return in_part<T, 2048, KIND, 8>(R, W);
-      // lengths 2^a m, m in {3, 5, 9, 25, 27, 125} (one register layout each)
+      // lengths 2^a m, m in {3, 5, 9, 25, 27, 125} (two register layouts each)
       case 12: return in_part<T, 12, KIND, 9>(R, W);
       case 18: return in_part<T, 18, KIND, 10>(R, W);
       case 20: return in_part<T, 20, KIND, 11>(R, W);
@@ -296,7 +304,7 @@ const void* by_n(int N, int R, int W) {
       case 1024: return in_part<T, 1024, KIND, 6>(R, W);
       case 2048: return in_part<T, 2048, KIND, 7>(R, W);
       case 4096: return in_part<T, 4096, KIND, 8>(R, W);
-      // nx = 2 M with M = 2^a m, m in {3, 5, 9, 25, 27, 125} (one register layout each)
+      // nx = 2 M with M = 2^a m, m in {3, 5, 9, 25, 27, 125} (two register layouts each)
       case 24: return in_part<T, 24, KIND, 9>(R, W);
       case 36: return in_part<T, 36, KIND, 10>(R, W);
       case 40: return in_part<T, 40, KIND, 11>(R, W);
