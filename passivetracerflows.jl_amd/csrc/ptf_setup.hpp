@@ -171,21 +171,22 @@ __global__ void layout_in_kernel(const double* __restrict__ src, T* __restrict__
   }
 }
 
-// Working layout (T, plus the low part when src_lo) -> public FP64 layout.
-template <typename T>
+// Values [first, last) of the public layout from the working layout (T, plus the low part
+// when src_lo), value i at dst[i - first].  OT is the type that crosses to the host: T where T
+// holds the whole value.  dst is pinned host memory: the stores go over the bus, contiguous.
+template <typename T, typename OT>
 __global__ void layout_out_kernel(const T* __restrict__ src, const T* __restrict__ src_lo,
-                                  double* __restrict__ dst, long long rows, int rowlen, int w,
-                                  int lb, int ndim, int ny) {
-  const long long n = rows * rowlen * w;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+                                  OT* __restrict__ dst, long long first, long long last, int rowlen,
+                                  int w, int lb, int ndim, int ny) {
+  for (long long i = first + (long long)blockIdx.x * blockDim.x + threadIdx.x; i < last;
        i += (long long)gridDim.x * blockDim.x) {
     const int e = (int)(i % w);
     const long long q = i / w;
     const long long k = q % rowlen, r = q / rowlen;
     const long long d = work_index(r, k, rowlen, lb, ndim, ny) * w + e;
-    double x = (double)src[d];
-    if (src_lo) x += (double)src_lo[d];
-    dst[i] = x;
+    OT x = (OT)src[d];
+    if (src_lo) x += (OT)src_lo[d];
+    dst[i - first] = x;
   }
 }
 
