@@ -10,7 +10,7 @@ template <int NX>
 const void* entry(int* threads) {
   constexpr int M = NX / 2, R = line_run_e(M);
   if constexpr (R > 0) {
-    *threads = M / R;
+    *threads = line_run_threads(M, R);
     return reinterpret_cast<const void*>(&line_run_kernel<PTF_T, NX, R, PTF_ETD != 0>);
   } else {
     return nullptr;
