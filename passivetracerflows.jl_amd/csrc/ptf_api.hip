@@ -2091,19 +2091,21 @@ int ptf_dealias(ptf_plan* plan, void* spec, double aliased_fraction) {
   if (!(aliased_fraction > 0.0)) return PTF_OK;   // [FF] dealias! does nothing then
   Group& g = plan->g;
   int rlo, rhi, ylo = 0, yhi = 0, zlo = 0, zhi = 0;
-  aliased_range(g.nx, aliased_fraction, &rlo, &rhi);
-  rhi = g.nxh;
+  aliased_range(g.nx, aliased_fraction, &rlo, &rhi);   // kr: to the end of the half axis
   if (g.ndim >= 2) aliased_range(g.ny, aliased_fraction, &ylo, &yhi);
   if (g.ndim == 3) aliased_range(g.nz, aliased_fraction, &zlo, &zhi);
-  const long long n = g.nS * g.B;
-  const int th = 256;
-  const unsigned blocks = (unsigned)std::min<long long>((n + th - 1) / th, 65536);
-  if (g.dbl)
-    hipLaunchKernelGGL(dealias_kernel<double>, dim3(blocks), dim3(th), 0, plan->stream,
-                       (cpx<double>*)spec, n, g.nxh, g.ny, g.nz, rlo, rhi, ylo, yhi, zlo, zhi);
-  else
-    hipLaunchKernelGGL(dealias_kernel<float>, dim3(blocks), dim3(th), 0, plan->stream,
-                       (cpx<float>*)spec, n, g.nxh, g.ny, g.nz, rlo, rhi, ylo, yhi, zlo, zhi);
+  // the kernel counts rows in 32 bits: members in chunks of at most 2^30 rows
+  const long long mrows = (long long)g.ny * g.nz, chunk = std::max(1LL, (1LL << 30) / mrows);
+  for (long long m = 0; m < g.B; m += chunk) {
+    const unsigned rows = (unsigned)(mrows * std::min<long long>(chunk, g.B - m));
+    const unsigned blocks = std::min((rows + 3) / 4, 16384u);
+    if (g.dbl)
+      hipLaunchKernelGGL(dealias_kernel<double>, dim3(blocks), dim3(256), 0, plan->stream,
+                         (cpx<double>*)spec + m * g.nS, rows, g.nxh, g.ny, g.nz, rlo, ylo, yhi, zlo, zhi);
+    else
+      hipLaunchKernelGGL(dealias_kernel<float>, dim3(blocks), dim3(256), 0, plan->stream,
+                         (cpx<float>*)spec + m * g.nS, rows, g.nxh, g.ny, g.nz, rlo, ylo, yhi, zlo, zhi);
+  }
   HIPCHK(hipGetLastError());
   return PTF_OK;
 }
@@ -2219,14 +2221,16 @@ static int set_analytic_impl(ptf_problem* prob, const ptf_flow_term* terms, int 
   a.ny = g.ny;
   a.nz = g.nz;
   a.lb = g.lb;
-  a.npoints = g.nR;
+  const long long len = (long long)(g.nx / 2) << g.lb;   // x-pairs of a group of 2^lb rows
+  a.parts = (int)((len + 255) / 256);
+  a.tiles = (unsigned)(g.nR / 2 / len * a.parts);
   Slot s;
   s.name = "flow_analytic_synthesis";
   s.dbl = g.dbl;
   s.kind = K_ANALYTIC;
   s.fn = reinterpret_cast<const void*>(&analytic_flow_kernel<T>);
   s.fixed_threads = 256;
-  s.fixed_blocks = (unsigned)std::min<long long>((g.nR + 255) / 256, 16384);
+  s.fixed_blocks = std::min(a.tiles, 16384u);
   set_args(s, a);
   bool tdep = false;
   for (int k = 0; k < nterms; ++k) tdep = tdep || terms[k].time_fn != PTF_FN_ONE;

@@ -194,6 +194,11 @@ __global__ void layout_out_kernel(const T* __restrict__ src, const T* __restrict
 // sum over the terms k of component c of ((amp[k] tx[k][ix]) ty[k][iy]) tz[k][iz]
 // (amp already holds amp * T(omega t + phase)).  Values are stored in the
 // library's physical layout: x-pairs, with the last axis in bricks of 2^lb rows.
+//
+// Bound by its stores: a flow that depends on time is written before every step.  A block
+// writes 256 consecutive x-pairs of one brick row (group: 2^lb rows that share their middle
+// index), so its indices come from one division a block and the stores of a wavefront are
+// contiguous.
 constexpr int kMaxFlowTerms = 16;
 template <typename T>
 struct AnalyticArgs {
@@ -205,60 +210,70 @@ struct AnalyticArgs {
   const double* tz;   // [nterms][nz]
   T* out[3];
   int ndim, nx, ny, nz, lb;
-  long long npoints;
+  int parts;          // blocks' worth of pairs in a group
+  unsigned tiles;     // groups * parts
 };
 
 template <typename T>
 __global__ void analytic_flow_kernel(AnalyticArgs<T> a) {
-  const long long B = 1ll << a.lb, mask = B - 1;
-  const long long mid = a.ndim == 3 ? a.ny : 1;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < a.npoints;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int ix = (int)(i % a.nx);
-    const long long r = i / a.nx;          // row: iy + ny iz
-    const int iy = a.ndim >= 2 ? (int)(r % a.ny) : 0;
-    const int iz = a.ndim == 3 ? (int)(r / a.ny) : 0;
-    double v0 = 0.0, v1 = 0.0, v2 = 0.0;
-    for (int k = 0; k < a.nterms; ++k) {
-      double x = a.amp[k] * a.tx[(long long)k * a.nx + ix];
-      if (a.ndim >= 2) x *= a.ty[(long long)k * a.ny + iy];
-      if (a.ndim == 3) x *= a.tz[(long long)k * a.nz + iz];
-      const int c = a.comp[k];
-      if (c == 0) v0 += x;
-      else if (c == 1) v1 += x;
-      else v2 += x;
+  const unsigned mask = (1u << a.lb) - 1;
+  const unsigned mid = a.ndim == 3 ? (unsigned)a.ny : 1u;
+  const unsigned len = ((unsigned)a.nx / 2) << a.lb;   // pairs of a group
+  for (unsigned tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+    const unsigned group = tile / (unsigned)a.parts, part = tile % (unsigned)a.parts;
+    const unsigned t = part * 256u + threadIdx.x;
+    if (t >= len) continue;
+    const unsigned last = ((group / mid) << a.lb) + (t & mask);   // index along the last axis
+    const int ix = 2 * (int)(t >> a.lb);
+    const int iy = a.ndim == 3 ? (int)(group % mid) : (int)last;
+    cpx<double> v[3] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+    // four terms at a time, so that their table reads are in flight together
+    for (int k0 = 0; k0 < a.nterms; k0 += 4) {
+      cpx<double> x[4];
+      double y[4], z[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = k0 + i < a.nterms ? k0 + i : a.nterms - 1;
+        const double* tx = a.tx + (long long)k * a.nx + ix;
+        x[i] = {tx[0], tx[1]};
+        y[i] = a.ndim >= 2 ? a.ty[(long long)k * a.ny + iy] : 0.0;
+        z[i] = a.ndim == 3 ? a.tz[(long long)k * a.nz + last] : 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (k0 + i >= a.nterms) break;
+        const double amp = a.amp[k0 + i];
+        x[i] = {amp * x[i].re, amp * x[i].im};
+        if (a.ndim >= 2) x[i] = {x[i].re * y[i], x[i].im * y[i]};
+        if (a.ndim == 3) x[i] = {x[i].re * z[i], x[i].im * z[i]};
+        const int c = a.comp[k0 + i];
+        if (c == 0) v[0] = v[0] + x[i];
+        else if (c == 1) v[1] = v[1] + x[i];
+        else v[2] = v[2] + x[i];
+      }
     }
-    // element ix of row r: pair ix/2 (bricked rows), component ix & 1
-    long long e;
-    const long long rowlen = a.nx / 2;
-    if (a.lb == 0) {
-      e = r * rowlen + ix / 2;
-    } else {
-      const long long l = r / mid, m = r % mid;
-      const long long b = ((l >> a.lb) * mid + m) * B + (l & mask);
-      e = ((b >> a.lb) * rowlen + ix / 2) * B + (b & mask);
-    }
-    const long long o = 2 * e + (ix & 1);
-    a.out[0][o] = (T)v0;
-    if (a.ndim >= 2) a.out[1][o] = (T)v1;
-    if (a.ndim == 3) a.out[2][o] = (T)v2;
+    const long long o = (long long)group * len + t;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (c < a.ndim) reinterpret_cast<cpx<T>*>(a.out[c])[o] = {(T)v[c].re, (T)v[c].im};
   }
 }
 
-// dealias!: zero the spectral elements whose kr index lies in [rlo, rhi) or whose
+// dealias!: zero the spectral elements whose kr index lies in [rlo, nxh) or whose
 // y (z) index lies in [ylo, yhi) ([zlo, zhi)); plain (unbricked) half-spectrum
-// layout (nx/2+1, ny, nz, batch), x fastest.
+// layout (nx/2+1, ny, nz, batch), x fastest.  A wavefront clears a row, so that the row's
+// place is found once and kept elements are not visited.
 template <typename T>
-__global__ void dealias_kernel(cpx<T>* __restrict__ f, long long n, int nxh, int ny, int nz,
-                               int rlo, int rhi, int ylo, int yhi, int zlo, int zhi) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int kx = (int)(i % nxh);
-    const long long r = i / nxh;
-    const int iy = (int)(r % ny);
-    const int iz = (int)((r / ny) % nz);
-    if ((kx >= rlo && kx < rhi) || (iy >= ylo && iy < yhi) || (iz >= zlo && iz < zhi))
-      f[i] = cpx<T>{(T)0, (T)0};
+__global__ void dealias_kernel(cpx<T>* __restrict__ f, unsigned rows, int nxh, int ny, int nz,
+                               int rlo, int ylo, int yhi, int zlo, int zhi) {
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lane = threadIdx.x % 64;
+  for (unsigned r = blockIdx.x * 4u + wave; r < rows; r += gridDim.x * 4u) {
+    const int iy = (int)(r % (unsigned)ny);
+    const int iz = (int)((r / (unsigned)ny) % (unsigned)nz);
+    const bool all = (iy >= ylo && iy < yhi) || (iz >= zlo && iz < zhi);
+    cpx<T>* row = f + (long long)r * nxh;
+    for (int k = (all ? 0 : rlo) + lane; k < nxh; k += 64) row[k] = cpx<T>{(T)0, (T)0};
   }
 }
 
