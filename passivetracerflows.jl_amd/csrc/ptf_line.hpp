@@ -215,7 +215,7 @@ void line_run_kernel(LineArgs<T> a) {
     for (int e = 0; e <= EP; ++e) x[e] = s[e];
     if constexpr (!ETD) {
       // as rk4_load / rk4_finish, the operands in registers: sp is the FP64 form's sol after
-      // the third stage
+      // the third stage; x_4 stays at hand, so its linear part joins in the fourth
       cpx<T> ac[EP + 1], sp[kMixed ? 1 : EP + 1];
 #pragma unroll 1
       for (int stage = 0; stage < 4; ++stage) {
@@ -233,7 +233,7 @@ void line_run_kernel(LineArgs<T> a) {
 #pragma unroll
             for (int e = 0; e <= EP; ++e) {
               const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
-              ac[e] = {ac[e].re / (T)6 + rhs.re / (T)3, ac[e].im / (T)6 + rhs.im / (T)3};
+              ac[e] = {div_by<6>(ac[e].re) + div_by<3>(rhs.re), div_by<6>(ac[e].im) + div_by<3>(rhs.im)};
               x[e] = {s[e].re + h2 * rhs.re, s[e].im + h2 * rhs.im};
             }
             break;
@@ -241,8 +241,8 @@ void line_run_kernel(LineArgs<T> a) {
 #pragma unroll
             for (int e = 0; e <= EP; ++e) {
               const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
-              ac[e] = {ac[e].re + rhs.re / (T)3, ac[e].im + rhs.im / (T)3};
               x[e] = {s[e].re + dt * rhs.re, s[e].im + dt * rhs.im};
+              ac[e] = {ac[e].re + div_by<3>(rhs.re), ac[e].im + div_by<3>(rhs.im)};
               if constexpr (!kMixed) sp[e] = {s[e].re + dt * ac[e].re, s[e].im + dt * ac[e].im};
             }
             break;
@@ -251,10 +251,10 @@ void line_run_kernel(LineArgs<T> a) {
             for (int e = 0; e <= EP; ++e) {
               const cpx<T> rhs = {N[e].re + L[e] * x[e].re, N[e].im + L[e] * x[e].im};
               if constexpr (!kMixed) {
-                s[e] = {sp[e].re + dt * (rhs.re / (T)6), sp[e].im + dt * (rhs.im / (T)6)};
+                s[e] = {sp[e].re + dt * div_by<6>(rhs.re), sp[e].im + dt * div_by<6>(rhs.im)};
                 if (a.st.filtered) s[e] = {(T)fil[e] * s[e].re, (T)fil[e] * s[e].im};
               } else {
-                const cpx<T> tot = {ac[e].re + rhs.re / (T)6, ac[e].im + rhs.im / (T)6};
+                const cpx<T> tot = {ac[e].re + div_by<6>(rhs.re), ac[e].im + div_by<6>(rhs.im)};
                 T hr, lr, hi, li;
                 comp_add(s[e].re, lo[e].re, dt * tot.re, hr, lr);
                 comp_add(s[e].im, lo[e].im, dt * tot.im, hi, li);
