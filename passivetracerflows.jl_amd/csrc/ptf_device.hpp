@@ -559,7 +559,7 @@ template <typename T>
 struct StageArgs {
   int kind;     // EPI_*
   int stage;    // 0..3
-  int store_x;  // RK4: also store the next stage's input in stg (its first transform
+  int store_x;  // also store the next stage's input in stg or stg2 (its first transform
                 // reads it from memory)
   cpx<T>* sol;  // state
   cpx<T>* sol_lo;  // mixed form: low part of the compensated state (sol + sol_lo), else NULL
@@ -657,6 +657,8 @@ __device__ __forceinline__ void comp_add(T hi, T lo, T y, T& ho, T& lo_out) {
 // ETDRK4 ([FF] ETDRK4substeps!/ETDRK4update!):
 //   sol1 = E2 sol + zeta N1 ; sol2 = E2 sol + zeta N2 ; sol2 = E2 sol1 + zeta (2 N3 - N1);
 //   sol = E sol + alpha N1 + 2 beta (N2 + N3) + Gamma N4
+// sol2 is the input of the third and then of the fourth stage and of nothing else: it is stored
+// only for a stage that transforms it from memory (store_x): two fields less written a step.
 // Every update returns the value it stores as the next stage's input (for the
 // last stage: the new sol), so a fused kernel can go on transforming it.
 
@@ -839,7 +841,7 @@ __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ub
         st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), v);
         st_pol<NTS>(lane_at<LEAN>(a.n1 + ubase, off), N);
       } else {
-        st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
+        if (a.store_x) st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
         st_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off), N);
       }
     }
@@ -852,7 +854,7 @@ __device__ __forceinline__ cpx<T> etd_finish(const StageArgs<T>& a, long long ub
     const double ai = o.e * o.si + o.al * (double)o.n1.im + be2 * ((double)o.n2.im + nim);
     const cpx<T> hi = {(T)ar, (T)ai};
     if (store) {
-      st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
+      if (a.store_x) st_pol<NTS>(lane_at<LEAN>(a.stg2 + ubase, off), v);
       st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), hi);
       if (kMixed && a.sol_lo)   // the low part of acc
         st_pol<NTS>(lane_at<LEAN>(a.n2 + ubase, off), {(T)(ar - (double)hi.re), (T)(ai - (double)hi.im)});

@@ -195,6 +195,9 @@ void col_kernel(ColArgs<T> a) {
   static_assert(epf_ok<MODE, EPF>(), "stage kernels take an epilogue family, others none");
   constexpr int P = N / R;
   constexpr bool kLean = fft_lean<T, R, OCC>();
+  // The unfused form's ETDRK4 stores take plain addresses: hipcc 7.2 fails on the scalar bases
+  // of its conditional stores ("illegal VGPR to SGPR copy", FP64 lines of 12 and more elements).
+  constexpr bool kLeanSt = kLean && MODE != COL_STAGE;
   // Non-temporal loads (and state stores) only where a block covers whole 128-byte lines
   // of a field: along the bricked axis a column's run is the 8 planes of a brick, so a
   // block reads TX * 8 consecutive elements; the columns of the 3D y pass are contiguous
@@ -421,7 +424,7 @@ void col_kernel(ColArgs<T> a) {
               const int ia = j + q * P;
               const int iky = a.axis == 2 ? by : ia;
               const int ikz = a.axis == 2 ? ia : iklast_col;
-              v[q] = etd_finish<T, ST, kNtS, kLean>(a.st, ub(q), off(q), ikx_col, iky, ikz, v[q], o[i], valid);
+              v[q] = etd_finish<T, ST, kNtS, kLeanSt>(a.st, ub(q), off(q), ikx_col, iky, ikz, v[q], o[i], valid);
             }
           }
         });
