@@ -219,7 +219,8 @@ struct Slot {
   int threads() const {
     if (fixed_threads > 0) return fixed_threads;
     if (is_col()) return W * (N / R);
-    return (par ? (kind == 14 ? 3 : 2) : 1) * W * ((N / 2) / R);
+    const int t = W * ((N / 2) / R);
+    return par ? (kind == 14 ? 3 : 2) * adv_par_group(t) : t;
   }
   dim3 grid() const {
     if (fixed_threads > 0) return dim3(fixed_blocks, 1, 1);
@@ -374,8 +375,13 @@ static Variant mixed_default(const Slot& s) {
   }
   const int W = narrow_width(L / en, 1);
   const bool adv = s.kind == K_ROW_ADV2 || s.kind == K_ROW_ADV3;
-  const int par = adv && (W * (L / en)) % 64 == 0 && !(s.kind == K_ROW_ADV3 && s.N > 128) &&
-                  !(!s.dbl && elems >= (1LL << 21));
+  // The rows side by side in groups that are not whole wavefronts: only in pairs, and in FP64
+  // only while a launch is latency (2D FP64 400 x 216 62 against 70 us a step, 500^2 92 against
+  // 100, 1000^2 164 against 172, but 1152^2 248 against 237; FP32 1152^2 175 against 178, 2000^2
+  // 564 against 590; three at a time 281 against 253 at 100^3 FP64).
+  const bool whole = (W * (L / en)) % 64 == 0;
+  const int par = adv && !(s.kind == K_ROW_ADV3 && (s.N > 128 || !whole)) &&
+                  elems < (s.dbl ? (whole ? 1LL << 62 : 1LL << 19) : 1LL << 21);
   return {en, W, 0, par, 0};
 }
 

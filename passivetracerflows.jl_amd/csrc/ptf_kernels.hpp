@@ -1013,8 +1013,13 @@ void row_kernel(RowArgs<T> a) {
 // of the block reaches every barrier and none ends early.  Compared with row_kernel
 // this trades idle lanes in the R2C for fewer registers per lane and all loads of a
 // block in flight together.
+//
+// A group is rounded up to whole wavefronts; the lanes beyond its rows repeat its last lane's
+// work (same loads, same values to the same places), so they need no case of their own.  A step
+// at 400 x 216 FP64, whose 4 rows of 20 lanes had no such form before: 70.1 -> 61.8 us.
+constexpr int adv_par_group(int lanes) { return (lanes + 63) / 64 * 64; }
 template <typename T, int NX, int R, int NL, int NIN>
-constexpr int adv_par_threads() { return NIN * NL * ((NX / 2) / R); }
+constexpr int adv_par_threads() { return NIN * adv_par_group(NL * ((NX / 2) / R)); }
 template <typename T, int NX, int R, int NL, int NIN>
 constexpr int adv_par_lds() { return NIN * NL * (NX / 2 + 1) * (int)sizeof(cpx<T>) + row_tw_bytes<T, NX>(); }
 
@@ -1028,8 +1033,7 @@ void row_adv_par_kernel(RowArgs<T> a) {
   constexpr int NXH = M + 1;
   constexpr int P = M / R;
   constexpr bool kLean = fft_lean<T, R, OCC>();
-  constexpr int G = NL * P;   // threads per group
-  static_assert(G % 64 == 0, "a group must be whole wavefronts");
+  constexpr int G = adv_par_group(NL * P);   // threads per group
   static_assert(NIN >= 2 && NIN <= 3, "two or three inputs");
   using Lay = LayStrided;
   const Lay lay = a.lb ? Lay{1, NL} : Lay{M + 1, 1};
@@ -1041,7 +1045,8 @@ void row_adv_par_kernel(RowArgs<T> a) {
     for (int i = (int)threadIdx.x; i < row_tw_elems<T, NX>(); i += (int)blockDim.x) twl[i] = a.tw[i * a.twstride];
   }
   const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / G);   // uniform over a wavefront
-  const int t = (int)threadIdx.x - grp * G;
+  int t = (int)threadIdx.x - grp * G;
+  if constexpr (G != NL * P) t = t < NL * P ? t : NL * P - 1;
   cpx<T>* lds = lds_all + grp * (NL * (M + 1));
   // lane and block mapping as in row_kernel
   const int lb = a.lb;

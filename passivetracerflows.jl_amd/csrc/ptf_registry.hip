@@ -112,9 +112,9 @@ const void* rowpar() {
     constexpr int NIN = row_nin(KIND);
     constexpr int M = NX / 2;
     constexpr int P = M / R;
-    constexpr bool ok = ((is_pow2_len(M) && R >= 4) || (R == line_e_narrow(M) && reduced_ok(M, R, NL, 16, P, OCC, KIND))) && R <= M &&
-                        (NL * P) % 64 == 0 &&
-                        NIN * NL * P <= 1024 &&
+    constexpr bool ok = ((is_pow2_len(M) && R >= 4 && (NL * P) % 64 == 0) ||
+                         (R == line_e_narrow(M) && reduced_ok(M, R, NL, 16, P, OCC, KIND))) && R <= M &&
+                        adv_par_threads<T, NX, R, NL, NIN>() <= 1024 &&
                         adv_par_lds<T, NX, R, NL, NIN>() <= 163840;
     if constexpr (ok) {
       return reinterpret_cast<const void*>(&row_adv_par_kernel<T, NX, R, NL, NIN, OCC>);
