@@ -72,6 +72,8 @@ def kernel_bytes(name: str, nS: int, nR: int, cb: int, rb: int, stage: int, step
     # The mixed form adds the low parts of its compensated pairs: ETDRK4 reads sol_lo in
     # stages 0-2, writes acc's low part in stage 2 and reads it in stage 3, writes sol_lo
     # in stage 3; RK4 stage 3 reads acc and sol_lo and writes sol_lo.
+    # The fused kernels leave out what no later stage reads from memory: RK4's write of x_4 in
+    # stage 2 and its read in stage 3, ETDRK4's two writes of sol2 (a step moves 2 S less).
     mixed = cb == 8
     if stepper.upper().endswith("ETDRK4"):
         state = {0: 3 * S + 2 * C, 1: 3 * S + 2 * C, 2: 6 * S + 5 * C, 3: 2 * S + C}[stage]

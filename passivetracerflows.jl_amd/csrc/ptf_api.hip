@@ -960,8 +960,8 @@ static bool build_member_slot(Group& g) {
 // 1D problems advance by whole runs of steps in one launch, a workgroup per member
 // (line_run_kernel), where a kernel is compiled for the length.  The four stage launches of a
 // step are kept for callers that time or select them one by one.  Always the faster of the
-// two: a step in a run takes 4.6 us against 23.6 by its four launches at 128 points FP64, 13
-// against 114 at 1000, 36 against 56 at 4096 (the nearest); FP32 ETDRK4 11 against 34 at 1024.
+// two: a step in a run takes 4.3 us against 23.6 by its four launches at 128 points FP64, 12
+// against 114 at 1000, 35 against 56 at 4096 (the nearest); FP32 ETDRK4 11 against 34 at 1024.
 // One step a call: 21 against 38 us at 128, 52 against 68 at 4096.
 template <typename T>
 static void build_line_slot(Group& g) {

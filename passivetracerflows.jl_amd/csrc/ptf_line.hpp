@@ -13,7 +13,7 @@
 // 17.5 us a step against 11).  Half of them are outside the transforms: the operators, the real
 // pre- and post-processing.  Where the transforms take up to 128 lanes those go to up to four
 // wavefronts, an element or two a lane, for two more exchanges a stage: 6.5 -> 4.6 us a step at
-// 128 points FP64, 25 -> 12.6 at 1000, 12 -> 10.8 at 1024 FP32 ETDRK4.
+// 128 points FP64 (4.3 with div_by), 25 -> 12.6 (12.2) at 1000, 12 -> 10.8 at 1024 FP32 ETDRK4.
 //
 // Per stage (calcN! S:695-710 for a steady 1D flow, then the stage update):
 //   N = R2C(-u C2R(i kr x))
