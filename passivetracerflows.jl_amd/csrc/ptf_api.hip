@@ -2537,7 +2537,7 @@ int ptf_step_record(ptf_problem* prob, int64_t nsteps, int64_t every, int64_t ca
   Group& g = prob->g;
   hipStream_t st = prob->stream;
   // records after the steps whose new clock.step is a multiple of `every`
-  auto floordiv = [](int64_t a, int64_t b) { return a >= 0 ? a / b : -((-a + b - 1) / b); };
+  auto floordiv = [](int64_t a, int64_t b) { return a / b - (a % b < 0 ? 1 : 0); };
   const int64_t s0 = prob->step;
   const int64_t nrec = floordiv(s0 + nsteps, every) - floordiv(s0, every);
   *nrec_out = nrec;
@@ -2553,8 +2553,9 @@ int ptf_step_record(ptf_problem* prob, int64_t nsteps, int64_t every, int64_t ca
   if (rc != PTF_OK) return rc;
   int64_t r = 0;
   for (int64_t left = nsteps; left > 0 && rc == PTF_OK;) {
-    // to the next record, or to the end
-    const int64_t n = std::min<int64_t>(left, every - ((prob->step % every) + every) % every);
+    // to the next record, or to the end (no sum with `every`, which may be the largest integer)
+    const int64_t past = prob->step % every;
+    const int64_t n = std::min<int64_t>(left, past < 0 ? -past : every - past);
     rc = step_direct(prob, n);
     if (rc != PTF_OK) break;
     left -= n;
