@@ -212,7 +212,9 @@ int ptf_autotune(ptf_problem* prob);
 /* Kernel-slot introspection for measurement: number of launches per step,
  * name of slot i, and the average duration of slot i over reps launches
  * (HIP events on the problem's stream).  Timing launches write only scratch
- * fields: the state is unchanged. */
+ * fields: the state is unchanged.  A 1D problem whose steps go to the whole-run
+ * kernel (PTF_VARIANT_RUN) lists the stage kernels that this kernel stands in
+ * for; time_slot times the listed kernel. */
 int ptf_problem_num_slots(ptf_problem* prob, int32_t* nslots);
 int ptf_problem_slot_name(ptf_problem* prob, int32_t slot, char* buf, int32_t buflen);
 int ptf_problem_time_slot(ptf_problem* prob, int32_t slot, int32_t reps, double* avg_ms);
@@ -223,14 +225,19 @@ int ptf_problem_time_slot(ptf_problem* prob, int32_t slot, int32_t reps, double*
  * (row slots) or the persistent pipelined stage kernel (fused column slots);
  * WG_LINES: a column line along the bricked axis spread over the workgroup with
  * workgroup barriers, where by default it is held by one wavefront (accepted only
- * for the slots and radices where the per-wavefront form applies). */
-enum { PTF_VARIANT_OCC3 = 1, PTF_VARIANT_PAR = 2, PTF_VARIANT_WG_LINES = 4 };
+ * for the slots and radices where the per-wavefront form applies).
+ * RUN (the stage slots of a 1D problem): runs of steps go to one launch of the
+ * whole-run kernel, the default where one is compiled for the length
+ * (ptf_autotune then has nothing to choose).  set_variant of a stage slot without
+ * it makes the stage kernels run, with it the whole-run kernel again. */
+enum { PTF_VARIANT_OCC3 = 1, PTF_VARIANT_PAR = 2, PTF_VARIANT_WG_LINES = 4, PTF_VARIANT_RUN = 8 };
 int ptf_problem_set_variant(ptf_problem* prob, int32_t slot, int32_t R, int32_t W, int32_t flags);
 int ptf_problem_get_variant(ptf_problem* prob, int32_t slot, int32_t* R, int32_t* W, int32_t* flags);
 /* ptf_step with a HIP event recorded around every launch of every step:
  * slot_ms[i] (num_slots entries) receives the average duration of slot i over
  * the nsteps steps, measured inside the running step sequence.  The state
- * advances exactly as with ptf_step. */
+ * advances exactly as with ptf_step.  Under PTF_VARIANT_RUN a step is one launch of
+ * the whole-run kernel: its duration is the first stage slot's, the others' are 0. */
 int ptf_step_profiled(ptf_problem* prob, int64_t nsteps, double* slot_ms);
 
 /* ---- ensembles: many independent 2D problems, one graph-captured launch

@@ -572,7 +572,7 @@ struct Group {
   std::vector<Slot> prologue;      // first inverse pass of a step when w0/w1 are not primed
   std::vector<Slot> stages[4];
   Slot line;                       // 1D: whole steps in one launch (fn null: none compiled)
-  bool use_line = false;           // off once a caller selects variants of the stage kernels
+  bool use_line = false;           // off where a caller selects the stage kernels (select_variant)
   std::vector<Slot> flowsyn;
   std::vector<ptf_flow_term> aterms;   // PTF_FLOW_ANALYTIC
   bool plan_only = false;              // a transform plan: no state, scratch for B members
@@ -1624,6 +1624,32 @@ static std::vector<Slot*> step_slots(Group& g) {
   return v;
 }
 
+// Whether the whole-run kernel does the work of this slot (a stage kernel of a 1D group).
+static bool run_stands_in(const Group& g, const Slot& s) { return g.use_line && s.kind == K_ROW_ADV1; }
+
+// The public variant of a slot of g, and the selection of one.  The stage kernels of a 1D group
+// are what runs after a selection without PTF_VARIANT_RUN, its whole-run kernel after one with it.
+static void variant_of(const Group& g, const Slot& s, int32_t* R, int32_t* W, int32_t* flags) {
+  *R = s.R;
+  *W = s.W;
+  *flags = (s.occ ? PTF_VARIANT_OCC3 : 0) | (s.par ? PTF_VARIANT_PAR : 0) | (s.wg ? PTF_VARIANT_WG_LINES : 0) |
+           (run_stands_in(g, s) ? PTF_VARIANT_RUN : 0);
+}
+static int select_variant(Group& g, Slot& s, int32_t R, int32_t W, int32_t flags) {
+  if (flags & ~(PTF_VARIANT_OCC3 | PTF_VARIANT_PAR | PTF_VARIANT_WG_LINES | PTF_VARIANT_RUN))
+    return fail(PTF_ERR_INVALID, "unknown flags");
+  const bool run = (flags & PTF_VARIANT_RUN) != 0;
+  Slot trial = s;
+  if ((run && (!g.line.fn || s.kind != K_ROW_ADV1)) ||
+      !choose_variant(trial, R, W, (flags & PTF_VARIANT_OCC3) ? 3 : 0, (flags & PTF_VARIANT_PAR) ? 1 : 0,
+                      (flags & PTF_VARIANT_WG_LINES) ? 1 : 0))
+    return fail(PTF_ERR_UNSUPPORTED, "no compiled variant R=" + std::to_string(R) + " W=" + std::to_string(W) +
+                                         " flags=" + std::to_string(flags) + " for slot " + s.name);
+  s = trial;
+  g.use_line = run;
+  return PTF_OK;
+}
+
 static int time_slot(Group& g, Slot& s, int reps, hipStream_t st, double* avg_ms) {
   if (reps < 1) reps = 1;
   g.primed = false;  // trial launches overwrite the transform scratch
@@ -1682,6 +1708,7 @@ struct TuneCand {
 };
 
 static int autotune_group(Group& g, hipStream_t st) {
+  if (g.use_line) return PTF_OK;   // no stage kernel runs, and the whole-run kernel has one form
   std::vector<Slot*> all = step_slots(g);
   std::vector<std::string> done;
   std::vector<std::pair<std::string, std::vector<TuneCand>>> shortlist;
@@ -2364,7 +2391,14 @@ int ptf_step_profiled(ptf_problem* prob, int64_t nsteps, double* slot_ms) {
   if (nsteps < 1) return fail(PTF_ERR_INVALID, "nsteps must be >= 1");
   Group& g = prob->g;
   hipStream_t st = prob->stream;
-  const std::vector<Slot*> v = step_slots(g);
+  std::vector<Slot*> v = step_slots(g);
+  for (size_t j = 0; j < v.size(); ++j) slot_ms[j] = 0.0;
+  if (g.use_line) {   // the whole-run kernel, a step a launch, in the place of the first stage kernel
+    v.resize(g.flowsyn.size());
+    if (g.dbl) args_of<LineArgs<double>>(g.line).nsteps = 1;
+    else args_of<LineArgs<float>>(g.line).nsteps = 1;
+    v.push_back(&g.line);
+  }
   const size_t ns = v.size();
   CHK(group_prime(g, st));
   // one event before the first launch and one after every launch of every step
@@ -2395,7 +2429,6 @@ int ptf_step_profiled(ptf_problem* prob, int64_t nsteps, double* slot_ms) {
   if (rc == PTF_OK && hipEventSynchronize(ev[k - 1]) != hipSuccess)
     rc = fail(PTF_ERR_DEVICE, "hipEventSynchronize");
   if (rc == PTF_OK) {
-    for (size_t j = 0; j < ns; ++j) slot_ms[j] = 0.0;
     for (size_t e = 1; e < k && rc == PTF_OK; ++e) {
       float ms = 0;
       if (hipEventElapsedTime(&ms, ev[e - 1], ev[e]) != hipSuccess)
@@ -2611,12 +2644,12 @@ int ptf_problem_num_slots(ptf_problem* prob, int32_t* n) {
   return PTF_OK;
 }
 
-static int slot_name_into(Slot& s, char* buf, int32_t buflen) {
+static int slot_name_into(const Group& g, const Slot& s, char* buf, int32_t buflen) {
   if (!buf || buflen <= 0) return fail(PTF_ERR_INVALID, "bad buffer");
   char tmp[256];
-  std::snprintf(tmp, sizeof(tmp), "%s [%s N=%d R=%d W=%d%s%s%s %s]", s.name.c_str(),
+  std::snprintf(tmp, sizeof(tmp), "%s [%s N=%d R=%d W=%d%s%s%s%s %s]", s.name.c_str(),
                 kind_name(s.kind), s.N, s.R, s.W, s.occ ? " occ=3" : "", s.par ? " par" : "",
-                s.wg ? " wg" : "", s.dbl ? "f64" : "f32");
+                s.wg ? " wg" : "", run_stands_in(g, s) ? " run" : "", s.dbl ? "f64" : "f32");
   std::strncpy(buf, tmp, (size_t)buflen - 1);
   buf[buflen - 1] = 0;
   return PTF_OK;
@@ -2626,7 +2659,7 @@ int ptf_problem_slot_name(ptf_problem* prob, int32_t slot, char* buf, int32_t bu
   if (!prob) return fail(PTF_ERR_INVALID, "problem is NULL");
   auto v = step_slots(prob->g);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  return slot_name_into(*v[slot], buf, buflen);
+  return slot_name_into(prob->g, *v[slot], buf, buflen);
 }
 
 int ptf_problem_time_slot(ptf_problem* prob, int32_t slot, int32_t reps, double* avg_ms) {
@@ -2640,16 +2673,7 @@ int ptf_problem_set_variant(ptf_problem* prob, int32_t slot, int32_t R, int32_t 
   if (!prob) return fail(PTF_ERR_INVALID, "problem is NULL");
   auto v = step_slots(prob->g);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  if (flags & ~(PTF_VARIANT_OCC3 | PTF_VARIANT_PAR | PTF_VARIANT_WG_LINES))
-    return fail(PTF_ERR_INVALID, "unknown flags");
-  Slot trial = *v[slot];
-  if (!choose_variant(trial, R, W, (flags & PTF_VARIANT_OCC3) ? 3 : 0,
-                      (flags & PTF_VARIANT_PAR) ? 1 : 0, (flags & PTF_VARIANT_WG_LINES) ? 1 : 0))
-    return fail(PTF_ERR_UNSUPPORTED, "no compiled variant R=" + std::to_string(R) +
-                                         " W=" + std::to_string(W) + " flags=" +
-                                         std::to_string(flags) + " for slot " + trial.name);
-  *v[slot] = trial;
-  prob->g.use_line = false;   // the caller's choice of stage kernels is what runs
+  CHK(select_variant(prob->g, *v[slot], R, W, flags));
   prob->drop_graph();
   return PTF_OK;
 }
@@ -2658,10 +2682,7 @@ int ptf_problem_get_variant(ptf_problem* prob, int32_t slot, int32_t* R, int32_t
   if (!prob || !R || !W || !flags) return fail(PTF_ERR_INVALID, "NULL argument");
   auto v = step_slots(prob->g);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  *R = v[slot]->R;
-  *W = v[slot]->W;
-  *flags = (v[slot]->occ ? PTF_VARIANT_OCC3 : 0) | (v[slot]->par ? PTF_VARIANT_PAR : 0) |
-           (v[slot]->wg ? PTF_VARIANT_WG_LINES : 0);
+  variant_of(prob->g, *v[slot], R, W, flags);
   return PTF_OK;
 }
 
@@ -2927,7 +2948,7 @@ int ptf_ensemble_slot_name(ptf_ensemble* ens, int32_t slot, char* buf, int32_t b
   if (!ens) return fail(PTF_ERR_INVALID, "ensemble is NULL");
   auto v = ens_slots(ens);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  return slot_name_into(*v[slot].second, buf, buflen);
+  return slot_name_into(*v[slot].first, *v[slot].second, buf, buflen);
 }
 
 int ptf_ensemble_time_slot(ptf_ensemble* ens, int32_t slot, int32_t reps, double* avg_ms) {
@@ -2941,16 +2962,7 @@ int ptf_ensemble_set_variant(ptf_ensemble* ens, int32_t slot, int32_t R, int32_t
   if (!ens) return fail(PTF_ERR_INVALID, "ensemble is NULL");
   auto v = ens_slots(ens);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  if (flags & ~(PTF_VARIANT_OCC3 | PTF_VARIANT_PAR | PTF_VARIANT_WG_LINES))
-    return fail(PTF_ERR_INVALID, "unknown flags");
-  Slot trial = *v[slot].second;
-  if (!choose_variant(trial, R, W, (flags & PTF_VARIANT_OCC3) ? 3 : 0,
-                      (flags & PTF_VARIANT_PAR) ? 1 : 0, (flags & PTF_VARIANT_WG_LINES) ? 1 : 0))
-    return fail(PTF_ERR_UNSUPPORTED, "no compiled variant R=" + std::to_string(R) +
-                                         " W=" + std::to_string(W) + " flags=" +
-                                         std::to_string(flags) + " for slot " + trial.name);
-  *v[slot].second = trial;
-  v[slot].first->use_line = false;
+  CHK(select_variant(*v[slot].first, *v[slot].second, R, W, flags));
   drop_graph(ens);
   return PTF_OK;
 }
@@ -2960,11 +2972,7 @@ int ptf_ensemble_get_variant(ptf_ensemble* ens, int32_t slot, int32_t* R, int32_
   if (!ens || !R || !W || !flags) return fail(PTF_ERR_INVALID, "NULL argument");
   auto v = ens_slots(ens);
   if (slot < 0 || slot >= (int)v.size()) return fail(PTF_ERR_INVALID, "slot out of range");
-  const Slot& s = *v[slot].second;
-  *R = s.R;
-  *W = s.W;
-  *flags = (s.occ ? PTF_VARIANT_OCC3 : 0) | (s.par ? PTF_VARIANT_PAR : 0) |
-           (s.wg ? PTF_VARIANT_WG_LINES : 0);
+  variant_of(*v[slot].first, *v[slot].second, R, W, flags);
   return PTF_OK;
 }
 

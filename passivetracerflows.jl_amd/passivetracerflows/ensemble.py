@@ -148,14 +148,23 @@ class Ensemble:
         sizes = ",".join(f"{c}x{n}^2" for n, c in sorted(Counter(self.sizes).items()))
         return f"ensemble {sizes} {self.precision} {self.stepper}"
 
-    def set_variant(self, i, R, W, occ3=False, par=False, wg=False):
-        call("ptf_ensemble_set_variant", self._h, i, R, W, variant_flags(occ3, par, wg))
+    def set_variant(self, i, R, W, occ3=False, par=False, wg=False, run=False):
+        """As Problem.set_variant, for launch slot i of the ensemble."""
+        call("ptf_ensemble_set_variant", self._h, i, R, W, variant_flags(occ3, par, wg, run))
+
+    def _variant(self, i):
+        R, W, f = C.c_int32(), C.c_int32(), C.c_int32()
+        call("ptf_ensemble_get_variant", self._h, i, C.byref(R), C.byref(W), C.byref(f))
+        return R.value, W.value, f.value
 
     def get_variant(self, i):
         """(R, W, occ3, par, wg) of launch slot i."""
-        R, W, f = C.c_int32(), C.c_int32(), C.c_int32()
-        call("ptf_ensemble_get_variant", self._h, i, C.byref(R), C.byref(W), C.byref(f))
-        return R.value, W.value, bool(f.value & 1), bool(f.value & 2), bool(f.value & 4)
+        R, W, f = self._variant(i)
+        return R, W, bool(f & 1), bool(f & 2), bool(f & 4)
+
+    def whole_run(self, i):
+        """Whether the whole-run kernel of a 1D group does the work of launch slot i."""
+        return bool(self._variant(i)[2] & 8)
 
     def slots(self):
         n = C.c_int32()

@@ -187,9 +187,9 @@ class DeviceArray:
             pass
 
 
-def variant_flags(occ3=False, par=False, wg=False):
-    """PTF_VARIANT_* bits: OCC3 = 1, PAR = 2, WG_LINES = 4 (include/ptf.h)."""
-    return (1 if occ3 else 0) | (2 if par else 0) | (4 if wg else 0)
+def variant_flags(occ3=False, par=False, wg=False, run=False):
+    """PTF_VARIANT_* bits: OCC3 = 1, PAR = 2, WG_LINES = 4, RUN = 8 (include/ptf.h)."""
+    return (1 if occ3 else 0) | (2 if par else 0) | (4 if wg else 0) | (8 if run else 0)
 
 
 def _devptr(a, shape=None, dtype=None, what="array"):
@@ -407,17 +407,26 @@ class Problem:
         call("ptf_problem_time_slot", self._h, i, reps, C.byref(ms))
         return ms.value
 
-    def set_variant(self, i, R, W, occ3=False, par=False, wg=False):
+    def set_variant(self, i, R, W, occ3=False, par=False, wg=False, run=False):
         """Select kernel variant (radix R, width W, 3-waves/SIMD build, input-parallel
         advection, bricked column lines spread over the workgroup) for launch slot i;
-        raises PTFError if it was not compiled or does not apply."""
-        call("ptf_problem_set_variant", self._h, i, R, W, variant_flags(occ3, par, wg))
+        raises PTFError if it was not compiled or does not apply.  A 1D problem then steps
+        with its stage kernels, or with the whole-run kernel again if run is set."""
+        call("ptf_problem_set_variant", self._h, i, R, W, variant_flags(occ3, par, wg, run))
+
+    def _variant(self, i):
+        R, W, f = C.c_int32(), C.c_int32(), C.c_int32()
+        call("ptf_problem_get_variant", self._h, i, C.byref(R), C.byref(W), C.byref(f))
+        return R.value, W.value, f.value
 
     def get_variant(self, i):
         """(R, W, occ3, par, wg) of launch slot i."""
-        R, W, f = C.c_int32(), C.c_int32(), C.c_int32()
-        call("ptf_problem_get_variant", self._h, i, C.byref(R), C.byref(W), C.byref(f))
-        return R.value, W.value, bool(f.value & 1), bool(f.value & 2), bool(f.value & 4)
+        R, W, f = self._variant(i)
+        return R, W, bool(f & 1), bool(f & 2), bool(f & 4)
+
+    def whole_run(self, i):
+        """Whether the whole-run kernel of a 1D problem does the work of launch slot i."""
+        return bool(self._variant(i)[2] & 8)
 
     def step_profiled(self, nsteps):
         """Advance nsteps steps (as stepforward_) with a HIP event around every launch;

@@ -35,18 +35,20 @@ def store(path, data):
 
 def apply_or_tune(obj, key, path, tune=None):
     """Apply the cached variants of ``key`` to ``obj`` (a Problem or an Ensemble: slots(),
-    set_variant(i, R, W, occ3, par, wg), get_variant(i)); if there is no matching entry, run the
-    autotuner (``tune``, default the object's own) and store its choice.  Returns "cache" or
-    "tuned"."""
+    set_variant(i, R, W, occ3, par, wg), get_variant(i), whole_run(i)); if there is no matching
+    entry, run the autotuner (``tune``, default the object's own) and store its choice.  Slots that
+    the whole-run kernel of a 1D problem stands in for keep it: the autotuner has no choice to make
+    there, and selecting a stage kernel would switch it off.  Returns "cache" or "tuned"."""
     data = load(path)
     names = [_base(n) for n in obj.slots()]
     entry = data.get(key)
+    whole_run = getattr(obj, "whole_run", lambda i: False)
     if entry and [e[0] for e in entry] == names:
         for i, e in enumerate(entry):
             R, W, occ3, par = e[1:5]
             wg = e[5] if len(e) > 5 else False
-            if int(R) == 0:
-                continue   # a fixed-shape kernel (whole-member step): nothing to select
+            if int(R) == 0 or whole_run(i):
+                continue   # a fixed-shape kernel (whole-member step, 1D run): nothing to select
             obj.set_variant(i, int(R), int(W), occ3=bool(occ3), par=bool(par), wg=bool(wg))
         return "cache"
     (tune or obj.autotune)()
