@@ -772,7 +772,7 @@ static StageArgs<T> stage_args(const Group& g, int stage) {
 template <typename T>
 static bool writes_sol(const StageArgs<T>& st) {
   if (st.kind == EPI_STORE) return false;
-  return st.stage == 3 || (st.kind == EPI_RK4 && st.stage == 2);
+  return st.stage == 3;
 }
 
 // The kernel kind of a stage's last column pass: with or without the fused first inverse

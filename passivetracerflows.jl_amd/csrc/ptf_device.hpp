@@ -647,13 +647,15 @@ __device__ __forceinline__ void comp_add(T hi, T lo, T y, T& ho, T& lo_out) {
 //   stage 2: acc = RHS_1/6 + RHS_2/3, stg = x_3;
 //   stage 3: x_4 is known here, so the linear part of RHS_4 joins the sum at once and x_4
 //            itself is stored only for a next stage that transforms it from memory
-//            (store_x): S = RHS_1/6 + RHS_2/3 + RHS_3/3 + L x_4/6; FP64 form: sol = sol +
-//            dt S, mixed form: acc = S (sol stays compensated);
-//   stage 4: FP64 form: sol = sol + dt N_4/6; mixed form: (sol, sol_lo) +=
+//            (store_x): acc = RHS_1/6 + RHS_2/3 + RHS_3/3 + L x_4/6;
+//   stage 4: FP64 form: sol += dt (acc + N_4/6); mixed form: (sol, sol_lo) +=
 //            dt (acc + N_4/6) with a compensated sum.
-// The FP64 form thus adds the last term to sol in two roundings instead of one.  Keeping x_4
-// out of memory saves a spectral field written and one read, 2 of the 26 that the stage kernels
-// of a step move (3D 256^3 FP64: stages 3 and 4 240 + 173 -> 196 + 136 us, a step 1.91 -> 1.83 ms).
+// sol takes one rounding a step.  The FP64 sum could go to sol in stage 3 and N_4/6 in stage 4,
+// a field less to move (256^3 FP64: 1876 us a step, 1905 this way), but the second rounding of the
+// state is the larger part of a step's error: 5.8e-16 against 4.5e-16 after 60 small steps from
+// a field of noise, 2.8e-16 against 2.6e-16 in a 400 x 216 filtered run of 80 steps.  Keeping x_4
+// out of memory saves a field written (FP64: 25 instead of 26 that the stage kernels of a step move;
+// mixed: a read as well).
 // ETDRK4 ([FF] ETDRK4substeps!/ETDRK4update!):
 //   sol1 = E2 sol + zeta N1 ; sol2 = E2 sol + zeta N2 ; sol2 = E2 sol1 + zeta (2 N3 - N1);
 //   sol = E sol + alpha N1 + 2 beta (N2 + N3) + Gamma N4
@@ -688,9 +690,9 @@ __device__ __forceinline__ Rk4Ops<T> rk4_load(const StageArgs<T>& a, long long u
   } else {
     if (stage == 2) o.x = ld_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off));
     o.s = ld_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off));
+    o.ac = ld_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off));
     // the compensated low part exists only in the mixed (FP32) form
     constexpr bool kMixed = sizeof(T) == 4;
-    if (stage == 2 || (kMixed && a.sol_lo)) o.ac = ld_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off));
     if (kMixed && stage == 3 && a.sol_lo) o.lo = ld_pol<NTS>(lane_at<LEAN>(a.sol_lo + ubase, off));
   }
   return o;
@@ -729,14 +731,13 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
     const cpx<T> tot = {o.ac.re + div_by<3>(rhs.re) + L6 * nx.re, o.ac.im + div_by<3>(rhs.im) + L6 * nx.im};
     if (store) {
       if (a.store_x) st_pol<NTS>(lane_at<LEAN>(a.stg + ubase, off), nx);
-      if (sizeof(T) == 4 && a.sol_lo) st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), tot);
-      else st_pol<NTS>(lane_at<LEAN>(a.sol + ubase, off), {o.s.re + dt * tot.re, o.s.im + dt * tot.im});
+      st_pol<NTS>(lane_at<LEAN>(a.acc + ubase, off), tot);
     }
     return nx;
   } else {
+    const cpx<T> tot = {o.ac.re + div_by<6>(N.re), o.ac.im + div_by<6>(N.im)};
     if (sizeof(T) == 8 || !a.sol_lo) {
-      // o.s = sol + dt S, stored by stage 3
-      cpx<T> ns = {o.s.re + dt * div_by<6>(N.re), o.s.im + dt * div_by<6>(N.im)};
+      cpx<T> ns = {o.s.re + dt * tot.re, o.s.im + dt * tot.im};
       if (a.filtered) {
         const T f = (T)filter_value(a.g, a.f_order, a.f_innerK, a.f_decay, ikx, iky, ikz);
         ns = {f * ns.re, f * ns.im};
@@ -745,7 +746,6 @@ __device__ __forceinline__ cpx<T> rk4_finish_L(const StageArgs<T>& a, long long 
       return ns;
     }
     // compensated accumulation: (hi, lo) += dt tot with TwoSum + renormalisation
-    const cpx<T> tot = {o.ac.re + div_by<6>(N.re), o.ac.im + div_by<6>(N.im)};
     T hr, lr, hi_, li_;
     comp_add(o.s.re, o.lo.re, dt * tot.re, hr, lr);
     comp_add(o.s.im, o.lo.im, dt * tot.im, hi_, li_);
