@@ -526,18 +526,97 @@ static int dalloc(DevBuf& b, size_t nbytes) {
   return PTF_OK;
 }
 
-// Pinned host memory that a field passes through on its way to the caller's array, in slots of
-// at most 2 MiB (kBounceSlots of them at most), each with the event that says it is filled.
+// Pinned host memory that a field passes through on its way to the caller's array: kBounceSlots
+// slots, each with the event that says it is filled.
 static constexpr int kBounceSlots = 8;
+static constexpr size_t kBounceSlotBytes = size_t(2) << 20;
 struct Bounce {
+  int dev = 0;   // the events' device
   void* p = nullptr;
-  size_t n = 0;
   hipEvent_t ev[kBounceSlots] = {};
   ~Bounce() {
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     if (p) (void)hipHostFree(p);
   }
+};
+
+// The sets are the process's, not a group's: pinning one and touching its pages takes up to 2.5 ms, as
+// long as four reads of a 1024^2 field, which a program may do once a problem; and many problems may
+// be alive.  A call has a set to itself while it runs, so threads and streams never share one.
+// ptf_device_init makes the first, as part of what a process does once (60 ms); at most kIdle sets a
+// device wait for the next call, one once no group is left, and the others are freed.  First read
+// of a new problem with a set a group: 128^2 FP64 128 us (later ones 28), 1024^2 1611 (373); so: 29, 390.
+class BouncePool {
+ public:
+  // null: no pinned memory to be had
+  std::unique_ptr<Bounce> take() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    {
+      std::lock_guard<std::mutex> l(m_);
+      for (size_t i = idle_.size(); i-- > 0;) {
+        if (idle_[i]->dev != dev) continue;
+        std::unique_ptr<Bounce> b = std::move(idle_[i]);
+        idle_.erase(idle_.begin() + (long)i);
+        return b;
+      }
+    }
+    std::unique_ptr<Bounce> b(new Bounce());
+    b->dev = dev;
+    bool ok = hipHostMalloc(&b->p, kBounceSlots * kBounceSlotBytes, hipHostMallocDefault) == hipSuccess;
+    if (ok) std::memset(b->p, 0, kBounceSlots * kBounceSlotBytes);   // the pages are there from here on
+    else b->p = nullptr;
+    for (auto& e : b->ev) {
+      if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        e = nullptr;
+        ok = false;
+      }
+    }
+    if (ok) return b;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  void give(std::unique_ptr<Bounce> b) {   // nothing of the call may be in flight in b any more
+    std::lock_guard<std::mutex> l(m_);
+    if (idle_of(b->dev) < (groups_ > 0 ? kIdle : 1)) idle_.push_back(std::move(b));
+  }
+  void group_made() {
+    std::lock_guard<std::mutex> l(m_);
+    ++groups_;
+  }
+  void group_gone() {
+    std::vector<std::unique_ptr<Bounce>> spare;
+    std::lock_guard<std::mutex> l(m_);
+    if (--groups_ > 0) return;
+    for (size_t i = idle_.size(); i-- > 0;) {
+      if (idle_of(idle_[i]->dev) < 2) continue;
+      spare.push_back(std::move(idle_[i]));
+      idle_.erase(idle_.begin() + (long)i);
+    }
+  }
+
+ private:
+  static constexpr size_t kIdle = 2;
+  size_t idle_of(int dev) const {
+    size_t n = 0;
+    for (auto& b : idle_) n += b->dev == dev;
+    return n;
+  }
+  std::mutex m_;
+  std::vector<std::unique_ptr<Bounce>> idle_;
+  long groups_ = 0;
+};
+// (never destroyed: the HIP runtime may be gone when static objects are)
+static BouncePool& bounce_pool() {
+  static BouncePool* pool = new BouncePool();
+  return *pool;
+}
+struct BounceUser {
+  BounceUser() { bounce_pool().group_made(); }
+  ~BounceUser() { bounce_pool().group_gone(); }
+  BounceUser(const BounceUser&) = delete;
+  BounceUser& operator=(const BounceUser&) = delete;
 };
 
 // blocks of the diagnostics' partial sums: Group::red holds a pair for each, and a record
@@ -547,6 +626,7 @@ static constexpr int kDiagBlocks = 1024;
 // group of B problems on one grid
 // ---------------------------------------------------------------------------
 struct Group {
+  BounceUser bounce_user;
   int ndim = 1, nx = 1, ny = 1, nz = 1, nxh = 1;
   int B = 1;
   int lb = 0;  // the last axis is stored in bricks of 2^lb planes (2D: y, 3D: z)
@@ -566,7 +646,6 @@ struct Group {
   std::vector<double> L_host;  // L in the public layout, all members
   DevBuf d_ops, sol, sol_lo, stg, stg2, acc, n1, n2, w[3], flow[3], d_L, etd[6], tw[3], psih0, omega;
   DevBuf stage;   // FP64 staging of one member in the public layout (fields from the host)
-  Bounce bounce;  // ... and the way of a field to the host
   DevBuf phys, spec, red, backup;  // set_c/updatevars/calcN staging, reductions, timing backup
   DevBuf fs[2];                    // spectral-flow synthesis scratch
   std::vector<Slot> prologue;      // first inverse pass of a step when w0/w1 are not primed
@@ -1458,31 +1537,11 @@ static int put_public(Group& g, bool dbl, void* dst, void* dst_lo, const double*
   return PTF_OK;
 }
 
-// Slots of a field of `nbytes`: one, or kBounceSlots of 64 KiB to 2 MiB.
+// Slots of a field of `nbytes`: one, or kBounceSlots of 64 KiB to kBounceSlotBytes.
 static size_t bounce_slot(size_t nbytes) {
   if (nbytes <= (size_t(512) << 10)) return nbytes;
   const size_t even = (nbytes / kBounceSlots + 4095) / 4096 * 4096;
-  return std::min(even, size_t(2) << 20);
-}
-
-// false: no pinned memory to be had
-static bool ensure_bounce(Group& g, size_t nbytes) {
-  Bounce& b = g.bounce;
-  const size_t need = std::min(nbytes, bounce_slot(nbytes) * kBounceSlots);
-  for (auto& e : b.ev) {
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-      e = nullptr;
-      (void)hipGetLastError();
-      return false;
-    }
-  }
-  if (b.p && b.n >= need) return true;
-  if (b.p) (void)hipHostFree(b.p);
-  b.n = need;
-  if (hipHostMalloc(&b.p, need, hipHostMallocDefault) == hipSuccess) return true;
-  b.p = nullptr;
-  (void)hipGetLastError();
-  return false;
+  return std::min(even, kBounceSlotBytes);
 }
 
 // values [first, last) of a field to dst, converted and reordered on the GPU
@@ -1506,14 +1565,15 @@ template <typename T, typename OT>
 static int get_public_t(Group& g, double* dst, const void* src, const void* src_lo,
                         long long rowlen, int w, hipStream_t st) {
   const long long n = (long long)g.ny * g.nz * rowlen * w;
-  if (!ensure_bounce(g, (size_t)n * sizeof(OT))) {
+  std::unique_ptr<Bounce> set = bounce_pool().take();
+  if (!set) {
     CHK(ensure_stage(g));
     HIPCHK((launch_out<T, double>(g, (double*)g.stage.p, src, src_lo, 0, n, rowlen, w, st)));
     HIPCHK(hipMemcpyAsync(dst, g.stage.p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     return PTF_OK;
   }
-  Bounce& b = g.bounce;
+  Bounce& b = *set;
   const long long per = (long long)(bounce_slot((size_t)n * sizeof(OT)) / sizeof(OT));
   const int chunks = (int)((n + per - 1) / per);
   auto slot = [&](int c) { return (OT*)b.p + c % kBounceSlots * per; };
@@ -1550,8 +1610,6 @@ static int get_public_t(Group& g, double* dst, const void* src, const void* src_
   if ((size_t)n * sizeof(double) < kBounceThreadBytes) {
     err = copier(0, 1);
   } else {
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
     hipError_t errs[kCopiers] = {};
     std::thread th[kCopiers];
     int started = 1;
@@ -1559,7 +1617,7 @@ static int get_public_t(Group& g, double* dst, const void* src, const void* src_
       const int h = started;
       try {
         th[h] = std::thread([&, h] {
-          errs[h] = hipSetDevice(dev);
+          errs[h] = hipSetDevice(b.dev);
           if (errs[h] == hipSuccess) errs[h] = copier(h, kCopiers);
         });
       } catch (const std::system_error&) {
@@ -1574,6 +1632,7 @@ static int get_public_t(Group& g, double* dst, const void* src, const void* src_
   }
   // the array is whole, or nothing of this call is left in flight
   const hipError_t se = hipStreamSynchronize(st);
+  if (se == hipSuccess) bounce_pool().give(std::move(set));   // else freed, which waits for the device
   HIPCHK(err);
   HIPCHK(se);
   return PTF_OK;
@@ -2002,6 +2061,7 @@ int ptf_device_init(int32_t ordinal) {
   HIPCHK(hipSetDevice(ordinal));
   void* scr = nullptr;
   CHK(static_scratch(ordinal, &scr));   // the allocation-free entry point's scratch address
+  if (std::unique_ptr<Bounce> set = bounce_pool().take()) bounce_pool().give(std::move(set));
   return PTF_OK;
 }
 
