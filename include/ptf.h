@@ -225,7 +225,8 @@ int ptf_problem_time_slot(ptf_problem* prob, int32_t slot, int32_t reps, double*
  * (row slots) or the persistent pipelined stage kernel (fused column slots);
  * WG_LINES: a column line along the bricked axis spread over the workgroup with
  * workgroup barriers, where by default it is held by one wavefront (accepted only
- * for the slots and radices where the per-wavefront form applies).
+ * for the slots and radices where the per-wavefront form applies, and for FP32 lines
+ * of 64 threads along that axis, which are always spread over the workgroup).
  * RUN (the stage slots of a 1D problem): runs of steps go to one launch of the
  * whole-run kernel, the default where one is compiled for the length
  * (ptf_autotune then has nothing to choose).  set_variant of a stage slot without

@@ -208,6 +208,7 @@ struct Slot {
     const int P = N / r;
     return P <= 64 && 64 % P == 0 && (dbl || P <= 32);
   }
+  // FP32 lines of 64 threads along a bricked axis: the workgroup form is the only one.
   bool wg_only(int r) const {
     return !dbl && is_col() && brick > 0 && fixed_threads == 0 && r > 0 && !((kind == 6 || kind == 8) && par) && N == 64 * r;
   }
@@ -246,7 +247,6 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
     // the workgroup form only where the wavefront one applies, or (FP32 lines of 64 threads)
     // where it is the only one
     if (!t.wave_ok(R) && !t.wg_only(R)) return false;
-    if (!t.wave_ok(R)) wg = 0;
   }
   if (s.brick > 0) {
     // a bricked line needs whole bricks per thread group; bricked rows go in whole bricks
@@ -1796,7 +1796,8 @@ static int autotune_group(Group& g, hipStream_t st) {
               bool ok = true;
               for (Slot* o : same) {
                 Slot trial = *o;
-                if (!choose_variant(trial, R, widths[wi], occ, par, wg) || trial.wg != wg) {
+                // (a line that has only the workgroup form needs no second timing of it)
+                if (!choose_variant(trial, R, widths[wi], occ, par, wg) || (wg && trial.wg_only(R))) {
                   ok = false;
                   break;
                 }
