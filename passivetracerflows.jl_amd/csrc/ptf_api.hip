@@ -1537,11 +1537,12 @@ static int put_public(Group& g, bool dbl, void* dst, void* dst_lo, const double*
   return PTF_OK;
 }
 
-// Slots of a field of `nbytes`: one, or kBounceSlots of 64 KiB to kBounceSlotBytes.
+// Slot size of a field of `nbytes`: an eighth of it, at least 512 KiB and at most kBounceSlotBytes.  A
+// slot costs a launch and an event, 10 us, so small ones cost more than the overlap gives: the
+// 528 KB spectrum of 256^2 FP64 takes 35 us in two slots and took 91 in eight (a pageable copy 48), 1.7 MB 92 against 117 (114).
 static size_t bounce_slot(size_t nbytes) {
-  if (nbytes <= (size_t(512) << 10)) return nbytes;
   const size_t even = (nbytes / kBounceSlots + 4095) / 4096 * 4096;
-  return std::min(even, kBounceSlotBytes);
+  return std::min(nbytes, std::min(std::max(even, size_t(512) << 10), kBounceSlotBytes));
 }
 
 // values [first, last) of a field to dst, converted and reordered on the GPU
