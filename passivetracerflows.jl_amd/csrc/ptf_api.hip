@@ -297,8 +297,13 @@ static Variant row_default(const Slot& s) {
   const long long rows = s.lines * s.members;
   const long long elems = rows * M, bytes = elems * (s.dbl ? 16 : 8);
   if (s.kind == K_ROW_C2R || s.kind == K_ROW_R2C) {
-    // contiguous rows need no wide blocks (256^3 FP32 inverse: 76 us at 4 rows, 89 at 8)
-    if (s.brick == 0) return s.N > 1024 ? Variant{8, 2, 0, 0, 0} : Variant{4, 4, 0, 0, 0};
+    // Contiguous rows need no wide blocks (256^3 FP32 inverse: 76 us at 4 rows, 89 at 8); rows of
+    // 4096 points one a block (a single one, FP64: 6.2 us, 8.6 at two a block of radix 8; 1024 of
+    // them 37 against 40 us), FP32 rows of 2048 that stream eight of radix 16 (2048 x 2048: 28
+    // against 31 us; a quarter of it 16 against 13).
+    if (s.brick == 0 && s.N > 2048) return {16, 1, 0, 0, 0};
+    if (s.brick == 0 && s.N > 1024) return !s.dbl && bytes >= (1LL << 24) ? Variant{16, 8, 0, 0, 0} : Variant{8, 2, 0, 0, 0};
+    if (s.brick == 0) return {4, 4, 0, 0, 0};
     if (s.N >= 1024) return {8, s.N >= 2048 ? 8 : 4, 0, 0, 0};
     return {4, s.N <= 256 ? 8 : 4, 0, 0, 0};
   }
@@ -337,6 +342,8 @@ static Variant col_default(const Slot& s) {
       return N < 64 || (N >= 256 && stream) ? Variant{4, 8, 0, 0, 0} : Variant{8, 8, 0, 0, 0};
     case K_COL_FWD:
     case K_COL_INV:
+      // (256 points FP32 streaming: the three passes of a 256^3 transform 73 us, 81 at radix 8)
+      if (!s.dbl && N == 256 && stream) return {16, 16, 0, 0, 0};
       return s.dbl || N <= 32 ? Variant{4, 8, 0, 0, 0} : Variant{8, 8, 0, 0, 0};
     case K_COL_FLOWSYN:
       return N >= 2048 ? Variant{8, 1, 0, 0, 0} : Variant{4, clampi(512 / N, 1, 8), 0, 0, 0};
