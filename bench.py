@@ -64,16 +64,16 @@ def kernel_bytes(name: str, nS: int, nR: int, cb: int, rb: int, stage: int, step
         return 2 * S + R + (2 * S if stage == 0 else 3 * S)
     if fam == "y_forward":
         return 2 * S
-    # RK4 state traffic of the FP64 form: stage 0 reads sol, writes acc; 1 reads sol, acc,
-    # writes stg, acc; 2 reads stg, sol, acc, writes stg, sol; 3 reads stg, sol, writes sol.
+    # RK4 state traffic of the FP64 form, the next stage's input stored: stage 0 reads sol,
+    # writes acc; 1 reads sol, acc, writes stg, acc; 2 reads stg, sol, acc, writes stg, acc; 3
+    # reads sol, acc, writes sol.
     # ETDRK4: 0 and 1 read sol, E2, zeta and write the next input and N; 2 reads sol, sol1,
     # N1, N2, E2, zeta, E, alpha, beta and writes sol2 and the partial update; 3 reads the
     # partial update and Gamma and writes sol.
     # The mixed form adds the low parts of its compensated pairs: ETDRK4 reads sol_lo in
     # stages 0-2, writes acc's low part in stage 2 and reads it in stage 3, writes sol_lo
-    # in stage 3; RK4 stage 3 reads acc and sol_lo and writes sol_lo.
-    # The fused kernels leave out what no later stage reads from memory: RK4's write of x_4 in
-    # stage 2 and its read in stage 3, ETDRK4's two writes of sol2 (a step moves 2 S less).
+    # in stage 3; RK4 stage 3 reads stg, acc and sol_lo and writes sol_lo.
+    # The fused kernels store and read less than that: see moved_bytes.
     mixed = cb == 8
     if stepper.upper().endswith("ETDRK4"):
         state = {0: 3 * S + 2 * C, 1: 3 * S + 2 * C, 2: 6 * S + 5 * C, 3: 2 * S + C}[stage]
@@ -95,6 +95,32 @@ def kernel_bytes(name: str, nS: int, nR: int, cb: int, rb: int, stage: int, step
     if fam.startswith("flow_x_c2r"):
         return S + R
     return None
+
+
+def moved_bytes(name: str, nS: int, nR: int, cb: int, rb: int, stage: int, stepper: str = "RK4"):
+    """Bytes of one launch as the fused schedule moves them: kernel_bytes without the fields that
+    no later stage reads from memory.  RK4 does not store x_4 (its linear part is in the sum that
+    stage 2 leaves) and the mixed form's stage 3 does not read it; ETDRK4 does not store sol2, the
+    input of stages 2 and 3, in stages 1 and 2."""
+    b = kernel_bytes(name, nS, nR, cb, rb, stage, stepper)
+    if b is None or not (name.startswith("stage") and name.split(" [")[0].endswith("_stage_inverse")):
+        return b
+    S = nS * cb
+    if stepper.upper().endswith("ETDRK4"):
+        return b - (S if stage in (1, 2) else 0)
+    return b - (S if stage == 2 or (stage == 3 and cb == 8) else 0)
+
+
+def kernel_source_hash():
+    """Hash of the device code of the step kernels, comments and white space aside: which code a
+    stored traffic measurement belongs to (a template name says only which variant)."""
+    import hashlib
+    import re
+    h = hashlib.sha256()
+    for f in ("ptf_device.hpp", "ptf_kernels.hpp"):
+        with open(os.path.join(ROOT, "passivetracerflows.jl_amd", "csrc", f)) as src:
+            h.update("".join(re.sub(r"//[^\n]*", "", src.read()).split()).encode())
+    return h.hexdigest()[:16]
 
 
 # kernel-kind name -> (template, MODE, DIR or NIN, epilogue family) of the HIP kernel it
@@ -205,7 +231,7 @@ def pmc_summary(fetch_dir, write_dir, cal_fetch_dir, cal_write_dir, bench_json):
                 tot += kib * 1024.0 * fac
         ent["hbm_bytes_per_launch"] = tot
         fams[fam] = ent
-    return dict(calibration=calib, families=fams,
+    return dict(kernel_source=kernel_source_hash(), calibration=calib, families=fams,
                 per_launch_bytes={f: e["hbm_bytes_per_launch"] for f, e in fams.items()})
 
 
@@ -398,7 +424,7 @@ def slot_table(prob, nS, nR, cb, rb, steps, stepper="RK4"):
     rows = []
     for i, (name, ms) in enumerate(zip(prob.slots(), prob.step_profiled(steps))):
         stage = int(name[5]) - 1 if name.startswith("stage") else 0
-        b = kernel_bytes(name, nS, nR, cb, rb, stage, stepper)
+        b = moved_bytes(name, nS, nR, cb, rb, stage, stepper)
         rows.append(dict(slot=i, name=name, ms=ms, bytes=b,
                          gbs=(b / (ms * 1e-3) / 1e9) if b else None))
     return rows
@@ -748,7 +774,7 @@ def main():
     step_ms_kernels = sum(r["ms"] for r in rows)
 
     # measured HBM bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a plain
-    # copy), used only when the measured kernel is the variant timed here
+    # copy), used only when the measured kernel is the variant timed here, of the same code
     traffic, traffic_variant = None, None
     tpath = os.path.join(ROOT, "profiles", "traffic_abc3d_256_fp64.json")
     if os.path.exists(tpath):
@@ -756,7 +782,7 @@ def main():
             tj = json.load(f)
         ent = tj.get("families", {}).get(dname, {})
         traffic_variant = ent.get("kernel_per_launch") or ent.get("kernel")
-        if ent.get("kernel_per_launch") == fam["templates"]:
+        if ent.get("kernel_per_launch") == fam["templates"] and tj.get("kernel_source") == kernel_source_hash():
             traffic = ent.get("hbm_bytes_per_launch")
 
     # mixed form of the same workload + its error against the FP64 run
