@@ -606,10 +606,12 @@ __device__ __forceinline__ double filter_value(const GridInfo& g, int order, dou
   return exp(-decay * ipow_d(K - innerK, order));
 }
 
-// x / D for a small whole D, correctly rounded (one Newton correction of x times the rounded
-// reciprocal: Markstein, "IA-64 and Elementary Functions", 2000, sect. 8.3; the last
-// instruction keeps the division's results for infinities, NaN and signed zeros).  4
-// instructions: the general division takes 11 and more, in one dependent chain.
+// x / D for a small whole D (one Newton correction of x times the rounded reciprocal: Markstein,
+// "IA-64 and Elementary Functions", 2000, sect. 8.3; the last instruction keeps the division's
+// results for infinities, NaN and signed zeros): correctly rounded where the quotient is a normal
+// number, within half a unit of the last place where it is subnormal (a tie there goes with the
+// rounding of 1/D instead of to even).  4 instructions: the general division takes 11 and
+// more, in one dependent chain.
 template <int D>
 __device__ __forceinline__ double div_by(double x) {
   constexpr double r = 1.0 / D;
