@@ -269,15 +269,15 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
 // ---- default variant -------------------------------------------------------------------
 // The variant a slot starts with (a problem runs with it unless ptf_autotune or a
 // set_variant call picks another).  For power-of-two lines it follows from the line length
-// and the size of the launch; the lines of the rule lie where the timings of every compiled
-// variant cross (33 problems: 1D 32..2048, 2D 64^2..2048^2 and oblong, 3D 32^3..256^3, batches
-// of members; the rule's choice is within 2 % of the fastest on average, 20 % at worst):
+// and the size of the launch; the lines of the rule lie where the timings of the compiled
+// variants cross.  Against what ptf_autotune picks (profiles/default_vs_tuned.md): 2D 64^2..2048^2 and
+// oblong, 3D 32^3..256^3, a step takes 1.00 of the tuned one's time on average, 1.06 at worst.
 //  * radix 4 while a launch has fewer wavefronts than the chip holds or a line is short: it
 //    gives the most threads per line (2D 256^2 FP64: x_advect 4.9 us against 35 us at radix
 //    16).  Long lines (rows from 1024, columns from 2048 points) and fields that stream from
 //    HBM take radix 8: fewer passes (3D 256^3 FP64 z kernel 134 us, radix 4 154 us).
 //  * the fewest lines per block that still fill a wavefront, so that a small field spreads
-//    over all CUs (256 of them); wider where there are blocks to spare, to read whole bricks
+//    over all CUs; wider where there are blocks to spare, to read whole bricks
 //    (rows: 4 of 8; 8 where a 3D field streams from HBM: 141 against 162 us at 256^3).
 //  * the 3-waves/SIMD build of the stage kernels where a launch is more than latency (FP32
 //    128^3 ETDRK4: 18 against 25 us), the default budget below (2D 256^2 FP32: 5.9 against 6.1).
@@ -287,7 +287,6 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
 struct Variant {
   int R, W, occ, par, wg;
 };
-static constexpr long long kCus = 256;
 
 static bool pow2_len(int n) { return n > 0 && (n & (n - 1)) == 0; }
 static int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -317,12 +316,12 @@ static Variant row_default(const Slot& s) {
   auto fits = [&](int W, int par) {
     const long long lds = (par ? nin : 1) * W * (M + 1) * cb + tw;
     const long long blocks = (rows + W - 1) / W;
-    return lds * (blocks > kCus ? 2 : 1) <= 163840;
+    return lds * (blocks > device_cus() ? 2 : 1) <= 163840;
   };
   int W = clampi(64 * R / M, 1, 16);
   int par = (W * (M / R)) % 64 == 0 && !(nin == 3 && s.N > 128) && !(!s.dbl && elems >= (1LL << 21)) && fits(W, 1);
   auto widen = [&]() {
-    while (W < (stream3 ? 8 : 4) && rows / (2 * W) >= kCus && fits(2 * W, par)) W *= 2;
+    while (W < (stream3 ? 8 : 4) && rows / (2 * W) >= device_cus() && fits(2 * W, par)) W *= 2;
   };
   widen();
   if (par && s.N >= 2048 && W < 2) {
@@ -368,7 +367,9 @@ static Variant col_default(const Slot& s) {
 // per lane do not spill, at the width that fills a wavefront, twice that where a field streams
 // (FP32 from 4 MB, FP64 from 64 MB: 200^3 stage kernels 56 against 85 us and 89 against 105).
 // Columns whose wide layout saves three passes or more (2^a 3 from 96 points on; FP32 also
-// 2^a 5, which spills in FP64) take it for fields from 16 MB: 192^3 FP64 54 against 65 us.
+// 2^a 5, which spills in FP64) take it for fields from 16 MB: 192^3 FP64 54 against 65 us.  Steps of
+// such grids take 1.08 of the tuned time on average (profiles/default_vs_tuned.md); lengths from 1100
+// points on and 768-point FP64 columns are where the rule is still off, by 10 to 45 %.
 static Variant mixed_default(const Slot& s) {
   const int L = s.is_col() ? s.N : s.N / 2;
   const int en = line_e_narrow(L), ew = line_e(L);
