@@ -6,7 +6,7 @@
 // `nsteps` whole steps in one launch: the state, the stage inputs, the operators and the flow
 // stay in registers, each thread holding elements j + q P (q < R) of the half-length line and
 // lane 0 the Nyquist element as well; LDS holds only the exchanges and the twiddle table.
-// Transforms of up to 64 lanes (256 points at radix 4) order their exchanges within one
+// Transforms of up to 64 lanes (lines of 512 points at radix 4) order their exchanges within one
 // wavefront, without workgroup barriers.  Radix 4 (6, 10, 3, 5 for the lengths that are no
 // powers of two): few elements per lane, since the time of a step is the instructions that one
 // wavefront issues one after the other (1024 points FP32 ETDRK4 in one wavefront of radix 8:
