@@ -549,12 +549,13 @@ struct Bounce {
   }
 };
 
-// The sets are the process's, not a group's: pinning one and touching its pages takes up to 2.5 ms, as
-// long as four reads of a 1024^2 field, which a program may do once a problem; and many problems may
-// be alive.  A call has a set to itself while it runs, so threads and streams never share one.
-// ptf_device_init makes the first, as part of what a process does once (60 ms); at most kIdle sets a
-// device wait for the next call, one once no group is left, and the others are freed.  First read
-// of a new problem with a set a group: 128^2 FP64 128 us (later ones 28), 1024^2 1611 (373); so: 29, 390.
+// The sets are the process's, not a group's: pinning one and the first touch of its pages take up to
+// 2.5 ms, as long as four reads of a 1024^2 field, which a program may do once a problem; and many
+// problems may be alive.  A call has a set to itself while it runs, so threads and streams never share
+// one.  ptf_device_init makes the first (0.3 ms of 60; the pages come with the reads that use them); at
+// most kIdle sets a device wait for the next call, one once no group is left, and the others are
+// freed.  First read of a new problem with a set a group: 128^2 FP64 128 us (later ones 28), 1024^2
+// 1611 (373); so: 29, 390.
 class BouncePool {
  public:
   // null: no pinned memory to be had
@@ -573,8 +574,7 @@ class BouncePool {
     std::unique_ptr<Bounce> b(new Bounce());
     b->dev = dev;
     bool ok = hipHostMalloc(&b->p, kBounceSlots * kBounceSlotBytes, hipHostMallocDefault) == hipSuccess;
-    if (ok) std::memset(b->p, 0, kBounceSlots * kBounceSlotBytes);   // the pages are there from here on
-    else b->p = nullptr;
+    if (!ok) b->p = nullptr;
     for (auto& e : b->ev) {
       if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
         e = nullptr;
