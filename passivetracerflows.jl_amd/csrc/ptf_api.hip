@@ -270,8 +270,8 @@ static bool choose_variant(Slot& s, int R, int W, int occ = 0, int par = 0, int 
 // The variant a slot starts with (a problem runs with it unless ptf_autotune or a
 // set_variant call picks another).  For power-of-two lines it follows from the line length
 // and the size of the launch; the lines of the rule lie where the timings of the compiled
-// variants cross.  Against what ptf_autotune picks (profiles/default_vs_tuned.md): 2D 64^2..2048^2 and
-// oblong, 3D 32^3..256^3, a step takes 1.00 of the tuned one's time on average, 1.06 at worst.
+// variants cross.  Against what ptf_autotune picks, 2D 64^2..2048^2 and oblong,
+// 3D 32^3..256^3, a step takes 1.00 of the tuned one's time on average, 1.06 at worst.
 //  * radix 4 while a launch has fewer wavefronts than the chip holds or a line is short: it
 //    gives the most threads per line (2D 256^2 FP64: x_advect 4.9 us against 35 us at radix
 //    16).  Long lines (rows from 1024, columns from 2048 points) and fields that stream from
@@ -368,7 +368,7 @@ static Variant col_default(const Slot& s) {
 // (FP32 from 4 MB, FP64 from 64 MB: 200^3 stage kernels 56 against 85 us and 89 against 105).
 // Columns whose wide layout saves three passes or more (2^a 3 from 96 points on; FP32 also
 // 2^a 5, which spills in FP64) take it for fields from 16 MB: 192^3 FP64 54 against 65 us.  Steps of
-// such grids take 1.08 of the tuned time on average (profiles/default_vs_tuned.md); lengths from 1100
+// such grids take 1.08 of the tuned time on average; lengths from 1100
 // points on and 768-point FP64 columns are where the rule is still off, by 10 to 45 %.
 static Variant mixed_default(const Slot& s) {
   const int L = s.is_col() ? s.N : s.N / 2;
